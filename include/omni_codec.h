@@ -484,8 +484,9 @@ int omni_snake_beta(const void* x, void* y, int dtype, int64_t batch, int64_t ch
  * Conv1d / ConvTranspose1d of channels-last activations in the general form of the reference's
  * channels-last conv API (sglang_omni/utils/channels_last_conv.py:45-120), for what the MFMA
  * kernel does not take: any channel counts, groups, stride, dilation and zero padding, float32,
- * bf16 or f16 activations, weights and bias of that dtype, float32 accumulation (taps ascending,
- * then the group's input channels), one rounding to the dtype:
+ * bf16 or f16 activations, weights and bias of that dtype, float32 accumulation in an order fixed by
+ * the shapes and strides (on the matrix cores where the groups are wide enough), one rounding to
+ * the dtype:
  *   conv        y[b, i, co] = bias[co] + sum_{j, c} W[co, c, j] x[b, i * stride + j * dilation -
  *               pad_left, g * C_in / groups + c]
  *   transposed  y[b, i, co] = bias[co] + sum_{j, c} W[g * C_in / groups + c, co - g * C_out /

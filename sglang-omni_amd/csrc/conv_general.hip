@@ -1,52 +1,20 @@
 // General Conv1d / ConvTranspose1d of channels-last activations: the shapes and dtypes of the
-// reference's channels-last conv API that the MFMA kernels do not take (channel counts that are
-// not multiples of 8 / 16, grouped and depthwise convs, any stride, dilation and zero padding,
-// float32 / fp16 activations). One thread per output element, float32 accumulation in a fixed
-// order (taps ascending, then the group's input channels ascending), rounded once.
+// reference's channels-last conv API that the packed bf16 MFMA kernels do not take (channel counts
+// that are not multiples of 8 / 16, grouped and depthwise convs, any stride, dilation and zero
+// padding, float32 / fp16 activations). Weights are read in the reference's own layout through
+// explicit strides ([C_out, C_in / g, k] for a conv, [C_in, C_out / g, k] for a transposed conv),
+// so callers pass the module's weight as it is.
 //
-// The thread's output channel is the fastest index, so a wave's threads read one input sample's
-// channels (broadcast or contiguous) and one weight column per tap; weights are read in the
-// reference's own layout through explicit strides ([C_out, C_in / g, k] for a conv, [C_in,
-// C_out / g, k] for a transposed conv), so callers pass the module's weight as it is.
-#include <type_traits>
-
-#include "common.h"
+// Groups of a few channels and more run on the matrix cores (conv_general_mfma.h, whose launcher
+// holds the rule). The rest (depthwise, very narrow groups) run here, one thread per output element: float32 accumulation in a
+// fixed order (taps ascending, then the group's input channels ascending), rounded once. The
+// thread's output channel is the fastest index, so a wave's threads read one input sample's
+// channels (broadcast or contiguous) and one weight column per tap.
+#include "conv_general.h"
 
 namespace {
 
-struct GeneralParams {
-  const void* x;
-  int64_t x_sb, x_st, x_sc;
-  int64_t batch, length_in, c_in;
-  const void* w;
-  int64_t w_s0, w_s1, w_s2, taps;
-  const void* bias;
-  int64_t c_out, groups, stride, dilation, pad_left;
-  void* y;
-  int64_t y_sb, y_st, y_sc, length_out;
-};
-
-template <typename T>
-__device__ __forceinline__ float load_as_float(const void* base, int64_t i) {
-  if constexpr (std::is_same<T, float>::value) {
-    return reinterpret_cast<const float*>(base)[i];
-  } else if constexpr (std::is_same<T, __bf16>::value) {
-    return bits_to_float_bf16(reinterpret_cast<const u16*>(base)[i]);
-  } else {
-    return bits_to_float_f16(reinterpret_cast<const u16*>(base)[i]);
-  }
-}
-
-template <typename T>
-__device__ __forceinline__ void store_from_float(void* base, int64_t i, float v) {
-  if constexpr (std::is_same<T, float>::value) {
-    reinterpret_cast<float*>(base)[i] = v;
-  } else if constexpr (std::is_same<T, __bf16>::value) {
-    reinterpret_cast<u16*>(base)[i] = float_to_bits_bf16(v);
-  } else {
-    reinterpret_cast<u16*>(base)[i] = float_to_bits_f16(v);
-  }
-}
+using namespace omni_general;
 
 template <typename T, bool TRANSPOSED>
 __global__ void __launch_bounds__(256) conv_general_kernel(const GeneralParams p) {
@@ -126,6 +94,10 @@ extern "C" int omni_conv1d_general(const void* x, int dtype, int64_t batch, int6
                   c_out, groups, stride, dilation, pad_left, y, y_stride_b, y_stride_t,
                   y_stride_c, length_out};
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const int status = dtype == OMNI_DTYPE_F32    ? launch_mfma_f32(p, transposed != 0, s)
+                     : dtype == OMNI_DTYPE_BF16 ? launch_mfma_bf16(p, transposed != 0, s)
+                                                : launch_mfma_f16(p, transposed != 0, s);
+  if (status != OMNI_ERR_UNSUPPORTED) return status;
   if (dtype == OMNI_DTYPE_F32) return launch_general<float>(p, transposed != 0, s);
   if (dtype == OMNI_DTYPE_BF16) return launch_general<__bf16>(p, transposed != 0, s);
   return launch_general<_Float16>(p, transposed != 0, s);
