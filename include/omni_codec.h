@@ -220,6 +220,11 @@ int omni_conv1d_fused(const omni_conv_args* args, omni_stream_t stream);
  *                                10 configurations
  *   OMNI_CONV_KERNEL_STAGED11    register-staged, taps <= 11, bf16 weights, x bf16; 10
  *   OMNI_CONV_KERNEL_FUSED_UNIT  the weight2 form (96 or 192 columns): full and short-row tiles
+ *   OMNI_CONV_KERNEL_SMALL       few positions (a streaming step of a few streams): bf16 operand
+ *                                used as is, bf16 weights, taps 1, 2 or 7: 9 configurations each
+ *                                (c_in a multiple of 96 for taps 1 and 2); the weight2 form at
+ *                                192 columns: 1. Taken for calls that leave the GPU mostly idle on
+ *                                the other families' tiles, with the same bits
  * omni_conv1d_fused_with runs the same arithmetic with the family and the list's config-th entry
  * (1-based) named by the caller (OMNI_ERR_UNSUPPORTED when they cannot serve the call); the
  * results of every configuration agree to float32 summation order. omni_conv1d_plan reports,
@@ -234,7 +239,8 @@ enum {
   OMNI_CONV_KERNEL_DMA = 1,
   OMNI_CONV_KERNEL_STAGED = 2,
   OMNI_CONV_KERNEL_STAGED11 = 3,
-  OMNI_CONV_KERNEL_FUSED_UNIT = 4
+  OMNI_CONV_KERNEL_FUSED_UNIT = 4,
+  OMNI_CONV_KERNEL_SMALL = 5
 };
 
 int omni_conv1d_fused_with(const omni_conv_args* args, int kernel, int config,

@@ -44,9 +44,11 @@ UNSUPPORTED = 2
 ABI_VERSION = 11
 
 # kernel families of omni_conv1d_fused (omni_conv1d_plan / omni_conv1d_fused_with)
-CONV_KERNEL_AUTO, CONV_KERNEL_DMA, CONV_KERNEL_STAGED, CONV_KERNEL_STAGED11, CONV_KERNEL_FUSED_UNIT = range(5)
+(CONV_KERNEL_AUTO, CONV_KERNEL_DMA, CONV_KERNEL_STAGED, CONV_KERNEL_STAGED11,
+ CONV_KERNEL_FUSED_UNIT, CONV_KERNEL_SMALL) = range(6)
 CONV_KERNEL_NAMES = {CONV_KERNEL_DMA: "dma", CONV_KERNEL_STAGED: "staged",
-                     CONV_KERNEL_STAGED11: "staged11", CONV_KERNEL_FUSED_UNIT: "fused_unit"}
+                     CONV_KERNEL_STAGED11: "staged11", CONV_KERNEL_FUSED_UNIT: "fused_unit",
+                     CONV_KERNEL_SMALL: "small"}
 
 
 class ConvArgs(ctypes.Structure):

@@ -115,3 +115,36 @@ def test_hifigan_resblock_convs_plan_to_their_tiles(channels, length, taps):
         # 32-column one-stage entry, which needs c_in = 32
         assert plan.config == (2 if channels == 64 else 1)
         assert plan.workgroups >= 256
+
+
+@pytest.mark.parametrize("layer", [
+    # a decoder layer at one stream of 4 frames, and at 64 streams of 12
+    ("block0.k7", 768, 768, 768, 7, 9, 32), ("block0.k1", 768, 768, 768, 1, 1, 32),
+    ("block0.up", 1536, 8 * 768, 768, 2, 1, 4), ("block1.k7", 384, 384, 384, 7, 3, 256),
+    ("block1.up", 768, 8 * 384, 384, 2, 1, 32), ("block2.k7", 192, 192, 192, 7, 9, 1280),
+])
+def test_small_calls_take_the_small_kernel_and_loaded_steps_do_not(layer):
+    name, c_in, n_cols, c_out, taps, d, positions = layer
+    kw = dict(c_in=c_in, n_cols=n_cols, c_out=c_out, taps=taps, dilation=d,
+              left_pad=1 if taps == 2 else None)
+    one = plan_shapes(batch=1, length=positions, **kw)
+    assert one.kernel == N.CONV_KERNEL_SMALL and one.configs == 9
+    assert plan_shapes(batch=64, length=positions * 3, **kw).kernel == N.CONV_KERNEL_DMA
+    # E4M3 weights and operands activated while staged keep their kernels
+    assert plan_shapes(batch=1, length=positions, fp8=True, **kw).kernel == N.CONV_KERNEL_DMA
+    act = plan_shapes(batch=1, length=positions, in_activation=N.ACT_SNAKE, **kw)
+    assert act.kernel == N.CONV_KERNEL_STAGED
+
+
+def test_what_no_tile_serves_the_small_kernel_does_not_either():
+    """The small kernel takes over calls that the large tiles serve, no others: many rows of two
+    samples with a wide halo fit no k = 7 tile and stay refused."""
+    kw = dict(batch=64, length=2, c_in=384, n_cols=384, c_out=384, taps=7, dilation=9)
+    with pytest.raises(N.OmniCodecError, match="status 2"):
+        plan_shapes(**kw)
+    unit = plan_shapes(batch=1, length=1280, c_in=192, n_cols=192, c_out=192, taps=7, dilation=9,
+                       fused_unit=True)
+    assert unit.kernel == N.CONV_KERNEL_SMALL and unit.configs == 1
+    loaded = plan_shapes(batch=64, length=3840, c_in=192, n_cols=192, c_out=192, taps=7,
+                         dilation=9, fused_unit=True)
+    assert loaded.kernel == N.CONV_KERNEL_FUSED_UNIT
