@@ -24,7 +24,8 @@
 //     reads meet no bank conflict either), E4M3 weights as bytes widened to bf16 (exactly) when
 //     read.
 //   * long rows (sweep): a workgroup runs consecutive tiles of one stream row, and each operand's
-//     last halo rows pass from one tile to the next through LDS instead of being recomputed.
+//     last halo rows pass from one tile to the next through LDS instead of being recomputed; where
+//     the sweep would leave most CUs idle, tiles of 256 or 128 staged rows recompute their halo.
 //   * streaming: rows left of position 0 of a stream row take each unit's own history copy (or
 //     zeros), and the workgroup that owns the last 6 * d positions of a row writes them as the
 //     unit's new history, as the one-unit kernel does.
@@ -485,9 +486,9 @@ __global__ void __launch_bounds__(64 * WCO * WP) residual_stack_kernel(const Sta
     // weight stage's barrier is that point; (a) and (b) below touch only rows that the dilated
     // conv reads after it
     stage_begin(k * Tile::STAGES);
-    // (a) operand rows left of position 0 (segments that start a stream row): the history copy
-    // of the row's slot, or zeros
-    if (i0 == 0 && h > 0) {
+    // (a) operand rows left of position 0 (the tile that starts a stream row, and short tiles
+    // whose halo reaches past it): the history copy of the row's slot, or zeros
+    if (i0 < H && h > 0) {
       for (int e = opaque_copy(tid); e < nseg * h * PIECES_PER_ROW; e += NT) {
         const int s = e / (h * PIECES_PER_ROW);
         const int rem = e - s * h * PIECES_PER_ROW;
@@ -502,8 +503,10 @@ __global__ void __launch_bounds__(64 * WCO * WP) residual_stack_kernel(const Sta
           }
         }
         const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(hr, off, 0, 0);
-        const int row = GUARD + s * span + H - h + j;
-        *reinterpret_cast<u32x4*>(us + uaddr<UROWS>(piece >> 2, row, piece & 3)) = v;
+        const int staged = H - h + j - i0;
+        if (staged >= 0)
+          *reinterpret_cast<u32x4*>(
+              us + uaddr<UROWS>(piece >> 2, GUARD + s * span + staged, piece & 3)) = v;
       }
       __syncthreads();
     }
@@ -756,9 +759,8 @@ __global__ void __launch_bounds__(64 * WCO * WP) residual_stack_kernel(const Sta
   if (p.fin_w != nullptr) {
     const int fh = p.fin_taps - 1;  // its causal context: staged rows H - fh .. H - 1
     const auto fr = buffer_rsrc(p.fin_hist, p.fin_hist_bytes);
-    // (a) context rows left of position 0 (segments that start a stream row): the history copy
-    // of the row's slot, or zeros
-    if (i0 == 0 && fh > 0) {
+    // (a) context rows left of position 0, as the units'
+    if (i0 < H && fh > 0) {
       for (int e = opaque_copy(tid); e < nseg * fh * PIECES_PER_ROW; e += NT) {
         const int s = e / (fh * PIECES_PER_ROW);
         const int rem = e - s * fh * PIECES_PER_ROW;
@@ -773,8 +775,10 @@ __global__ void __launch_bounds__(64 * WCO * WP) residual_stack_kernel(const Sta
           }
         }
         const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(fr, off, 0, 0);
-        const int row = GUARD + s * span + H - fh + j;
-        *reinterpret_cast<u32x4*>(us + uaddr<UROWS>(piece >> 2, row, piece & 3)) = v;
+        const int staged = H - fh + j - i0;
+        if (staged >= 0)
+          *reinterpret_cast<u32x4*>(
+              us + uaddr<UROWS>(piece >> 2, GUARD + s * span + staged, piece & 3)) = v;
       }
     }
     __syncthreads();
@@ -883,14 +887,39 @@ using Stack96Dma = StackTile<96, 1, 8, 3>;
 using Stack96Sweep = StackTile<96, 1, 8, 3, true>;
 using Stack96Dma8 = StackTile<96, 1, 8, 3, false, true>;
 using Stack96Sweep8 = StackTile<96, 1, 8, 3, true, true>;
+// The tiled form at 256 and 128 staged rows (2 and 1 position tiles a wave), for calls that give
+// the sweep few workgroups.
+template <int TP, bool W8>
+using Stack96Tiled = StackTile<96, 1, 8, TP, false, W8>;
 static_assert(Stack96Sweep::lds_bytes() <= 160 * 1024, "the sweep form fits the CU's LDS");
 static_assert(Stack96Sweep8::lds_bytes() <= Stack96Sweep::lds_bytes() &&
               Stack96Dma8::R == Stack96Dma::R && Stack96Sweep8::R == Stack96Dma::R,
               "E4M3 weights take the bf16 forms' tiles");
 
+// How a launch stages its rows: the sweep, or tiles of 384, 256 or 128 staged rows.
+enum StackForm { kFormSweep, kForm384, kForm256, kForm128 };
+
+template <int TP, bool W_FP8, bool SWEEP>
+int launch_stack_form(const StackParams& p, int grid, hipStream_t stream) {
+  using Tile = StackTile<96, 1, 8, TP, SWEEP, W_FP8>;
+  auto k = residual_stack_kernel<96, 1, 8, TP, W_FP8, SWEEP>;
+  static const bool raised = omni_conv::raise_lds_limit((const void*)k);
+  (void)raised;
+  hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(Tile::NT), Tile::lds_bytes(), stream, p);
+  OMNI_LAUNCH_CHECK();
+  return OMNI_OK;
+}
+
 template <bool W_FP8>
-int launch_stack96(const StackParams& p, int grid, bool sweep, hipStream_t stream);
-template <> int launch_stack96<false>(const StackParams& p, int grid, bool sweep, hipStream_t stream);
-template <> int launch_stack96<true>(const StackParams& p, int grid, bool sweep, hipStream_t stream);
+int launch_stack96(const StackParams& p, int grid, StackForm form, hipStream_t stream) {
+  switch (form) {
+    case kFormSweep: return launch_stack_form<3, W_FP8, true>(p, grid, stream);
+    case kForm384: return launch_stack_form<3, W_FP8, false>(p, grid, stream);
+    case kForm256: return launch_stack_form<2, W_FP8, false>(p, grid, stream);
+    default: return launch_stack_form<1, W_FP8, false>(p, grid, stream);
+  }
+}
+extern template int launch_stack96<false>(const StackParams&, int, StackForm, hipStream_t);
+extern template int launch_stack96<true>(const StackParams&, int, StackForm, hipStream_t);
 
 }  // namespace omni_stack

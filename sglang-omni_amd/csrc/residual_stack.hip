@@ -217,6 +217,7 @@ extern "C" int omni_residual_stack(const omni_residual_stack_args* a, omni_strea
   // the staged rows need, evened out; short rows as many whole rows (each with its halo) as the
   // staged rows hold.
   int64_t grid;
+  StackForm form = kForm384;
   bool sweep = false;
   if (L + H > R && a->num_units <= kSweepUnits) {
     int64_t halo_rows = fin ? a->final_taps - 1 : 0;
@@ -244,6 +245,28 @@ extern "C" int omni_residual_stack(const omni_residual_stack_args* a, omni_strea
     p.sweep_segments = (int)segments;
     p.sweep_positions = (int)((L + segments - 1) / segments);
     grid = B * segments;
+    form = kFormSweep;
+    // Few positions give the sweep few workgroups, each running two and more tiles one after the
+    // other (56 to 65 us each): smaller tiles, each with the whole stack's halo, spread them over the
+    // GPU. Measured, us, sweep / 256 rows / 128 rows: 1 x 7 680 positions 129 / 40 / 29, 1 x
+    // 23 040 130 / 41 / 80, 8 x 7 680 131 / 79 / 152, 16 x 7 680 131 / 117 / 275, 1 x 480 000 279
+    // / 412 / 1 060.
+    const int64_t tiles = (p.sweep_positions + R - 1) / R;
+    double least = 64.0 * tiles;
+    const struct { StackForm form; int64_t rows; double us; } small[] = {
+        {kForm256, Stack96Tiled<2, false>::R, 40.0}, {kForm128, Stack96Tiled<1, false>::R, 28.0}};
+    for (const auto& f : small) {
+      if (H + 32 > f.rows) continue;
+      const int64_t per_row = (L + (f.rows - H) - 1) / (f.rows - H);
+      const double us = f.us * ((B * per_row + cus - 1) / cus);
+      if (us < least) {
+        least = us;
+        form = f.form;
+        p.seg_len = (int)((L + per_row - 1) / per_row);
+        p.tiles_per_row = (int)((L + p.seg_len - 1) / p.seg_len);
+        grid = B * p.tiles_per_row;
+      }
+    }
   } else if (L + H > R) {
     const int64_t tiles = (L + (R - H) - 1) / (R - H);
     p.seg_len = (int)((L + tiles - 1) / tiles);
@@ -257,6 +280,6 @@ extern "C" int omni_residual_stack(const omni_residual_stack_args* a, omni_strea
   }
   if (grid > 0x7fffffffLL) return OMNI_ERR_UNSUPPORTED;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  return fp8 ? launch_stack96<true>(p, (int)grid, sweep, s)
-             : launch_stack96<false>(p, (int)grid, sweep, s);
+  return fp8 ? launch_stack96<true>(p, (int)grid, form, s)
+             : launch_stack96<false>(p, (int)grid, form, s);
 }

@@ -220,3 +220,36 @@ def test_residual_stack_precomputed_coefficients_give_the_same_bits(gpu, fp8, di
     with pytest.raises(ValueError):
         residual_stack(x, units, torch.empty_like(outs[0][0]), out_a, out_b,
                        coef_table=table[:-1])
+
+
+@pytest.mark.parametrize("batch,length", [
+    (1, 301), (1, 345), (1, 4000),       # 128 staged rows: the halo of the first tiles past position 0
+    (1, 12000), (3, 5000), (16, 1500),   # 256 staged rows
+    (100, 2000), (1, 100001),            # the sweep: three tiles a workgroup, an odd length
+])
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("cold", [True, False])
+def test_every_form_of_long_rows_equals_one_launch_per_unit(gpu, batch, length, fp8, cold):
+    """The forms the launcher picks by size, with slot histories read (or zeros) and written."""
+    units, out_a, out_b = make_units((1, 3, 9), gpu, fp8=fp8, seed=11)
+    gen = torch.Generator(device=gpu).manual_seed(length)
+    x = (torch.randn(batch, length, C, generator=gen, device=gpu) * 0.3).half()
+    pools = [torch.randn(batch, 2, 6 * d, C, generator=gen, device=gpu).bfloat16() for d in (1, 3, 9)]
+    index = torch.arange(batch, device=gpu).flip(0).contiguous()
+    parity = torch.arange(batch, device=gpu) % 2
+    kw = dict(slot_index=index, slot_parity=parity, history_cold=cold)
+    out = torch.empty(batch, length, C, dtype=torch.bfloat16, device=gpu)
+    got = [p.clone() for p in pools]
+    residual_stack(x, units, out, out_a, out_b, histories=got, **kw)
+    want = [p.clone() for p in pools]
+    ref = x.float()
+    u = identity_operand(ref, units[0].in_a, units[0].in_b)
+    for k, unit in enumerate(units):
+        a, b = (units[k + 1].in_a, units[k + 1].in_b) if k < 2 else (out_a, out_b)
+        nxt, total = torch.empty_like(u), torch.empty_like(ref)
+        fused_conv(u, unit.conv1, nxt, second=unit.conv2, mid_activation=N.ACT_SNAKE,
+                   mid_a=unit.mid_a, mid_b=unit.mid_b, residual=ref, sum_out=total,
+                   activation=N.ACT_SNAKE, act_a=a, act_b=b, history=want[k], **kw)
+        u, ref = nxt, total
+    assert torch.equal(out, u)
+    assert all(torch.equal(p, q) for p, q in zip(got, want))
