@@ -1,8 +1,8 @@
 // HiFT's short-time Fourier transform and its inverse (the iSTFT tail of the CosyVoice3 /
-// MiniCPM-o vocoders), on gfx950. Both are HBM-bound: a 16-point transform does 16 MACs per
-// output component, so the kernels read their input once, keep the small bases and the
-// workgroup's window of frames in LDS, and give every output one fixed summation order (so a row's
-// result does not depend on the batch or the tiling). HiFT's geometry (n_fft 16, hop 4) has its
+// MiniCPM-o vocoders), on gfx950. Both are near HBM-bound: a 16-point transform does 16 MACs per
+// output component, so the kernels read their input once, keep the workgroup's window of frames
+// in LDS, and give every output one fixed summation order (so a row's result does not depend on
+// the batch or the tiling). HiFT's geometry (n_fft 16, hop 4) has its
 // own instantiation with the loops unrolled; other sizes take the runtime-sized kernels.
 //
 //   short_time_spectrum: spectrum[r, c, f] = sum_{k < n_fft} x[r, f * hop + k - pad] * basis[c, k]
@@ -214,97 +214,184 @@ __global__ void __launch_bounds__(kThreads) overlap_add_inverse_kernel(const Ist
   p.out[row * p.out_stride + i] = y;
 }
 
-// HiFT's geometry (n_fft 16, hop 4, 9 bins): each thread finishes 4 samples of one window phase
-// r = sample % 4 (samples i0 + tid + 256 k), so its 4 x 18 basis values and 4 squared-window
-// values stay in registers for all of them (2 or 8 samples per thread measured slower: 8 leaves
-// each workgroup's exp / sin / sincos staging too long a serial chain); the workgroup's frames sit in LDS as rows of 20
-// floats (18 components, 2 pad) read 16 bytes at a time. Every output takes the generic kernel's
-// terms in its order (overlaps ascending, then bins), so the two give the same bits.
-constexpr int kInv16Samples = 4 * kThreads;  // samples per workgroup
-constexpr int kInv16Pitch = 20;              // floats per frame row in LDS
-constexpr int inverse16_frames() { return (kInv16Samples - 1) / 4 + 16 / 4 + 1; }
-constexpr size_t inverse16_lds_bytes() { return (size_t)inverse16_frames() * kInv16Pitch * 4; }
+// The tail's exp, sin and cos. The general library functions took 27 of the tail's 44 us (every
+// call carries its argument's whole range reduction and, for sine and cosine, both polynomials);
+// these keep float32 accuracy (a unit in the last place, as those do) in fewer instructions.
 
+// exp(x): 2^(x log2 e) with the product's rounding error and log2 e's own put back. x is clamped to
+// where exp is 0 or infinite beyond; NaN gives what the caller's clip makes of infinity.
+__device__ __forceinline__ float tail_exp(float x) {
+  x = fmaxf(fminf(x, 150.f), -150.f);
+  const float hi = x * 1.4426950216293335f;
+  const float lo = __builtin_fmaf(x, 1.925963033500011e-08f,
+                                  __builtin_fmaf(x, 1.4426950216293335f, -hi));
+  const float e = __builtin_amdgcn_exp2f(hi);
+  return __builtin_fmaf(e, lo * 0.6931471824645996f, e);
+}
+
+// sin(x): x - k pi in three fused steps (pi as three floats), an odd polynomial on [-pi/2, pi/2]
+// (least maximum relative error, 5e-9, fitted with the leading coefficient fixed at 1), the sign of
+// k's parity. Beyond 2^15, and for infinities and NaN, the library's.
+__device__ __forceinline__ float tail_sin(float x) {
+  if (!(fabsf(x) < 32768.f)) return sinf(x);
+  const float k = rintf(x * 0.31830987334251404f);
+  float r = __builtin_fmaf(-k, 3.1415927410125732f, x);
+  r = __builtin_fmaf(-k, -8.742277657347586e-08f, r);
+  r = __builtin_fmaf(-k, -3.4302490200117637e-15f, r);
+  const float z = r * r;
+  float q = __builtin_fmaf(z, 2.6087894e-06f, -0.00019811053f);
+  q = __builtin_fmaf(z, q, 0.008333088f);
+  q = __builtin_fmaf(z, q, -0.1666666f);
+  r = __builtin_fmaf(r * z, q, r);
+  return __uint_as_float(__float_as_uint(r) ^ ((uint32_t)(int)k << 31));
+}
+
+// sin and cos of p in [-1, 1] (a sine's value): polynomials fitted there (5e-11 and 1e-9).
+__device__ __forceinline__ void tail_sincos(float p, float& sn, float& cs) {
+  const float z = p * p;
+  float q = __builtin_fmaf(z, 2.6953126e-06f, -0.00019836212f);
+  q = __builtin_fmaf(z, q, 0.008333317f);
+  q = __builtin_fmaf(z, q, -0.16666667f);
+  sn = __builtin_fmaf(p * z, q, p);
+  float c = __builtin_fmaf(z, 2.4215466e-05f, -0.0013884914f);
+  c = __builtin_fmaf(z, c, 0.041666582f);
+  c = __builtin_fmaf(z, c, -0.5f);
+  cs = __builtin_fmaf(z, c, 1.f);
+}
+
+// HiFT's geometry (n_fft 16, hop 4, 9 bins), 1 024 samples a workgroup. The window's frames go to
+// LDS as rows of 18 components (the tail's input first as it lies in memory, coalesced, then each
+// (frame, bin) pair replaced by its real and imaginary part); each 16 frames are transformed on the
+// matrix cores (v_mfma_f32_16x16x4_f32, float32 products and sums: D[t][frame] over 20 components,
+// two of them zero), which leaves a lane the four consecutive values 4 o .. 4 o + 3 of one frame:
+// what that frame adds to the four samples of the quad o hops later. The quads' four parts meet
+// through LDS, overlaps ascending, and leave as 16-byte stores. Before, every sample read its four
+// frames' 72 components from LDS (16 us of LDS traffic at the size below) and multiplied them on
+// the VALU. An output's sum order is fixed: components in the MFMA's order within a frame, then
+// overlaps. Bound by: the tail's VALU work per (frame, bin), about 40 instructions; the inverse, HBM.
+// Measured, 16 x 240 000 samples: tail 43.8 -> 26.1 us (84 MB: 3.2 TB/s), inverse 50.4 -> 23.4 us
+constexpr int kInv16Quads = kThreads;                  // quads of samples per workgroup
+constexpr int kInv16Samples = 4 * kInv16Quads;
+constexpr int kInv16Frames = kInv16Quads + 3;          // frames that reach them
+constexpr int kInv16Groups = (kInv16Frames + 15) / 16;  // MFMA groups of 16 frames
+
+template <bool TAIL>
 __global__ void __launch_bounds__(kThreads) overlap_add_inverse16_kernel(const IstftParams p) {
-  constexpr int NF = 16, HP = 4, BINS = 9, COMPS = 18, OV = NF / HP, HALF = NF / 2;
-  extern __shared__ float smem[];
-  float* spec = smem;  // [frames of the window][kInv16Pitch]
-  const int tid = threadIdx.x;
+  constexpr int NF = 16, BINS = 9, COMPS = 18, OV = 4, ROWS = kInv16Groups * 16;
+  // the spectra, then (once every wave holds its groups' results) the quads' parts [OV][ROWS]: one
+  // buffer, so eight workgroups share a CU
+  __shared__ __attribute__((aligned(16))) float spec[ROWS * COMPS];
+  static_assert(OV * ROWS * 4 <= ROWS * COMPS, "the parts fit the spectra's buffer");
+  f32x4* parts = reinterpret_cast<f32x4*>(spec);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t row = blockIdx.y;
   const int64_t i0 = (int64_t)blockIdx.x * kInv16Samples;
-  const int64_t fa = (i0 + HALF) / HP - (OV - 1);
-  const int64_t fb = (i0 + kInv16Samples - 1 + HALF) / HP;
-  const int nf = (int)(fb - fa + 1);
-  if (p.tail) {
-    for (int e = tid; e < nf * BINS; e += kThreads) {
-      const int j = e / BINS;
-      const int b = e - j * BINS;
-      const int64_t f = fa + j;
-      float re = 0.f, im = 0.f;
-      if (f >= 0 && f < p.frames) {
-        const float* hf = p.h + row * p.h_row_stride + f * p.h_frame_stride;
-        const float mag = fminf(expf(hf[b]), p.mag_clip);
-        const float phase = sinf(hf[BINS + b]);
-        float sn, cs;
-        sincosf(phase, &sn, &cs);
-        re = mag * cs;
-        im = mag * sn;
+  const int64_t q0 = i0 / 4 + 2;  // the first quad: padded position / 4
+  const int64_t fa = q0 - (OV - 1);
+  // the window's frames inside the row: lo .. hi - 1 of its kInv16Frames
+  const int lo = fa < 0 ? (int)-fa : 0;
+  const int hi = (int)min((int64_t)kInv16Frames, p.frames - fa);
+  if constexpr (TAIL) {
+    const float* hr = p.h + row * p.h_row_stride + fa * p.h_frame_stride;
+    if (p.h_frame_stride == COMPS && (reinterpret_cast<uintptr_t>(hr) & 7) == 0) {
+      // packed frames: one run of memory, 8 bytes a load, all in flight together
+      constexpr int N = kInv16Frames * COMPS / 2, U = (N + kThreads - 1) / kThreads;
+      const uint2* src = reinterpret_cast<const uint2*>(hr);
+      uint2 v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int e = tid + u * kThreads;
+        v[u] = e >= lo * (COMPS / 2) && e < hi * (COMPS / 2) ? src[e] : uint2{0u, 0u};
       }
-      spec[j * kInv16Pitch + b] = re;
-      spec[j * kInv16Pitch + BINS + b] = im;
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (tid + u * kThreads < N) reinterpret_cast<uint2*>(spec)[tid + u * kThreads] = v[u];
+    } else {
+      for (int e = lo * COMPS + tid; e < hi * COMPS; e += kThreads) {
+        const int j = e / COMPS;
+        spec[e] = hr[j * p.h_frame_stride + (e - j * COMPS)];
+      }
+    }
+    __syncthreads();
+    int j = tid / BINS, b = tid - j * BINS;
+#pragma unroll 3
+    for (int e = tid; e < kInv16Frames * BINS; e += kThreads) {
+      float* s = spec + j * COMPS + b;
+      const float mag = fminf(tail_exp(s[0]), p.mag_clip);
+      float sn, cs;
+      tail_sincos(tail_sin(s[BINS]), sn, cs);
+      const bool real = j >= lo && j < hi;
+      s[0] = real ? mag * cs : 0.f;
+      s[BINS] = real ? mag * sn : 0.f;
+      j += kThreads / BINS;
+      b += kThreads % BINS;
+      if (b >= BINS) b -= BINS, ++j;
     }
   } else {
-    for (int e = tid; e < nf * COMPS; e += kThreads) {
-      const int j = e / COMPS;
-      const int c = e - j * COMPS;
-      const int64_t f = fa + j;
-      float v = 0.f;
-      if (f >= 0 && f < p.frames) {
+    // component c's run of frames, a thread's frames of every component in flight together
+    const int64_t first = row * BINS * p.frames + fa;
+    for (int j = tid; j < kInv16Frames; j += kThreads) {
+      float v[COMPS];
+      const bool real = j >= lo && j < hi;
+#pragma unroll
+      for (int c = 0; c < COMPS; ++c) {
         const float* src = c < BINS ? p.re : p.im;
-        const int b = c < BINS ? c : c - BINS;
-        v = src[(row * BINS + b) * p.frames + f];
+        v[c] = real ? src[first + (c % BINS) * p.frames + j] : 0.f;
       }
-      spec[j * kInv16Pitch + c] = v;
+#pragma unroll
+      for (int c = 0; c < COMPS; ++c) spec[j * COMPS + c] = v[c];
     }
   }
-  // this thread's window phase (i0 is a multiple of HP): t = r + HP o for overlap o
-  const int r = (tid + HALF) % HP;
-  float bas[OV][COMPS], w2[OV];
+  // operand lanes: output t (or frame) lane % 16, component 4 s + lane / 16 of step s
+  const int ln = lane & 15, lq = lane >> 4;
+  float basis[5];
 #pragma unroll
-  for (int o = 0; o < OV; ++o) {
-    w2[o] = p.win2[r + HP * o];
+  for (int s = 0; s < 5; ++s) basis[s] = 4 * s + lq < COMPS ? p.basis[(4 * s + lq) * NF + ln] : 0.f;
+  __syncthreads();
+  constexpr int GROUPS = (kInv16Groups + kThreads / 64 - 1) / (kThreads / 64);  // of a wave
+  f32x4 acc[GROUPS];
 #pragma unroll
-    for (int c = 0; c < COMPS; ++c) bas[o][c] = p.basis[c * NF + r + HP * o];
+  for (int k = 0; k < GROUPS; ++k) {
+    acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int g = wave + k * (kThreads / 64);
+    if (g >= kInv16Groups) break;
+    const float* sp = spec + (g * 16 + ln) * COMPS + lq;
+#pragma unroll
+    for (int s = 0; s < 5; ++s) {
+      const float v = s < 4 || lq < 2 ? sp[4 * s] : 0.f;  // components 18 and 19 do not exist
+      acc[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(basis[s], v, acc[k], 0, 0, 0);
+    }
   }
   __syncthreads();
-#pragma unroll 1
-  for (int k = 0; k < kInv16Samples / kThreads; ++k) {
-    const int64_t i = i0 + tid + (int64_t)k * kThreads;
-    if (i >= p.samples) break;
-    const int64_t pos = i + HALF;
-    float signal = 0.f, envelope = 0.f;
 #pragma unroll
-    for (int o = 0; o < OV; ++o) {
-      const int64_t f = pos / HP - o;
-      if (f < 0 || f >= p.frames) continue;
-      const f32x4* sv = reinterpret_cast<const f32x4*>(spec + (int)(f - fa) * kInv16Pitch);
-      float s[kInv16Pitch];
+  for (int k = 0; k < GROUPS; ++k) {
+    const int g = wave + k * (kThreads / 64);
+    if (g < kInv16Groups) parts[lq * ROWS + g * 16 + ln] = acc[k];
+  }
+  __syncthreads();
+  const int64_t i = i0 + 4 * tid;
+  if (i >= p.samples) return;  // samples come in whole quads: hop * (frames - 1)
+  f32x4 signal = f32x4{0.f, 0.f, 0.f, 0.f}, envelope = signal;
 #pragma unroll
-      for (int q = 0; q < kInv16Pitch / 4; ++q) {
-        const f32x4 v = sv[q];
-        s[4 * q] = v[0];
-        s[4 * q + 1] = v[1];
-        s[4 * q + 2] = v[2];
-        s[4 * q + 3] = v[3];
-      }
+  for (int o = 0; o < OV; ++o) {
+    const int64_t f = q0 + tid - o;
+    if (f < 0 || f >= p.frames) continue;
+    signal += parts[o * ROWS + tid + OV - 1 - o];
 #pragma unroll
-      for (int b = 0; b < BINS; ++b)
-        signal += __builtin_fmaf(s[b], bas[o][b], s[BINS + b] * bas[o][BINS + b]);
-      envelope += w2[o];
-    }
-    float y = signal / envelope;
-    if (p.tail) y = fminf(fmaxf(y, -p.audio_limit), p.audio_limit);
-    p.out[row * p.out_stride + i] = y;
+    for (int r = 0; r < 4; ++r) envelope[r] += p.win2[4 * o + r];
+  }
+  float* out = p.out + row * p.out_stride + i;
+  f32x4 y;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    y[r] = signal[r] / envelope[r];
+    if (TAIL) y[r] = fminf(fmaxf(y[r], -p.audio_limit), p.audio_limit);
+  }
+  if ((reinterpret_cast<uintptr_t>(out) & 15) == 0) {
+    *reinterpret_cast<f32x4*>(out) = y;
+  } else {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) out[r] = y[r];
   }
 }
 
@@ -363,8 +450,8 @@ int launch_inverse(IstftParams& p, int64_t rows, omni_stream_t stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (p.n_fft == 16 && p.hop == 4) {
     dim3 grid16((unsigned)((p.samples + kInv16Samples - 1) / kInv16Samples), (unsigned)rows);
-    hipLaunchKernelGGL(overlap_add_inverse16_kernel, grid16, dim3(kThreads), inverse16_lds_bytes(),
-                       s, p);
+    hipLaunchKernelGGL(p.tail ? overlap_add_inverse16_kernel<true> : overlap_add_inverse16_kernel<false>,
+                       grid16, dim3(kThreads), 0, s, p);
   } else {
     hipLaunchKernelGGL((overlap_add_inverse_kernel<0, 0>), grid, dim3(kThreads), lds, s, p);
   }

@@ -1,0 +1,73 @@
+"""The iSTFT tail's own exp, sine and cosine over their ranges, and its frame windows at their edges,
+against float64.
+
+Bound: an output is a sum of 4 x 18 products of magnitude * cos / sin with the basis over the
+envelope, each factor within 4 float32 roundings (exp, sine of a sine, product) and the sums within
+72 more, relative to the sum of the absolute terms."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from oracle import codec_oracle as O
+from sglang_omni_amd.kernels.hift import HiftStft, overlap_add_inverse
+
+pytestmark = pytest.mark.gpu
+
+
+def parts(h):
+    h = h.double()
+    mag, phase = torch.exp(h[..., :9]).clamp(max=100.0), torch.sin(h[..., 9:18])
+    return (mag * torch.cos(phase)).transpose(1, 2), (mag * torch.sin(phase)).transpose(1, 2)
+
+
+# one frame more than a workgroup's window of quads, one less, ragged, one sample quad
+@pytest.mark.parametrize("frames", [2, 255, 256, 257, 258, 511, 514, 1003])
+@pytest.mark.parametrize("phase_scale", [1.0, 300.0, 3e4, 1e6])
+@pytest.mark.parametrize("layout", ["packed", "wide", "unaligned"])
+def test_tail_against_float64(gpu, frames, phase_scale, layout):
+    gen = torch.Generator().manual_seed(frames)
+    h = torch.randn(3, frames, 18, generator=gen)
+    h[..., :9] = h[..., :9] * 0.8 - 4.0
+    h[..., 9:] *= phase_scale
+    h[0, :, 0] = torch.linspace(-140.0, 2.0, frames)  # magnitudes down to zero
+    h[1, :, 9] = torch.pi * torch.arange(frames).float()  # sines near zero
+    st = HiftStft(O.hann_window(16), 4, device=gpu)
+    hd = h.to(gpu)
+    if layout == "wide":  # rows of 20 channels, the last two not read
+        hd = torch.cat([hd, torch.full((3, frames, 2), float("nan"), device=gpu)], dim=2)
+    elif layout == "unaligned":  # a view whose first element is 4 bytes past an 8-byte boundary
+        flat = torch.empty(3 * frames * 18 + 1, device=gpu)
+        flat[1:] = hd.reshape(-1)
+        hd = flat[1:].view(3, frames, 18)
+    re, im = parts(h)
+    want = O.istft_reference(re, im, O.hann_window(16), 16, 4).clamp(-0.99, 0.99)
+    scale = float(torch.maximum(re.abs(), im.abs()).amax())
+    got = st.tail(hd).cpu()
+    assert got.shape == want.shape
+    err = (got.double() - want).abs().max().item()
+    # 18 components of at most `scale`, basis at most 2 / 16, over 4 frames and an envelope >= 1.49
+    assert err <= (4 + 72) * 2.0 ** -24 * 4 * 18 * scale * (2 / 16) / 1.49
+    # the inverse over the same parts, rounded to float32 first
+    inv = overlap_add_inverse(re.float().contiguous().to(gpu), im.float().contiguous().to(gpu),
+                              st.inverse_basis, st.squared_window, 4).cpu()
+    full = O.istft_reference(re, im, O.hann_window(16), 16, 4)
+    assert (inv.double() - full).abs().max().item() <= 74 * 2.0 ** -24 * 9 * scale / 1.49
+
+
+def test_tail_at_the_ends_of_the_range(gpu):
+    """Infinite magnitudes clip, vanishing ones are zero, and a NaN or infinite phase marks the
+    samples of its frame's window and no other."""
+    st = HiftStft(O.hann_window(16), 4, device=gpu)
+    h = torch.full((1, 400, 18), -3.0)
+    h[..., 9:] = 0.5
+    h[0, 100, 3], h[0, 101, 4], h[0, 102, 5] = float("inf"), float("-inf"), 1e30
+    re, im = parts(h)
+    want = O.istft_reference(re, im, O.hann_window(16), 16, 4).clamp(-0.99, 0.99)
+    torch.testing.assert_close(st.tail(h.to(gpu)).cpu().double(), want, rtol=1e-5, atol=1e-5)
+    for bad in (float("nan"), float("inf")):
+        h[0, 200, 12] = bad
+        nan = st.tail(h.to(gpu)).cpu().isnan()[0].nonzero().flatten().tolist()
+        # frame 200 covers samples 792 .. 807; clamping a NaN sample gives a limit, as before
+        assert all(792 <= i < 808 for i in nan)
