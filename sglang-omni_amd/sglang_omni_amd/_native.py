@@ -288,7 +288,7 @@ def check(status: int, what: str) -> None:
 def require_device(*tensors: torch.Tensor) -> None:
     """The kernels run on the GPU only: refuse CPU tensors instead of falling back."""
     for t in tensors:
-        if t is not None and t.device.type != "cuda":
+        if t is not None and not t.is_cuda:
             raise OmniCodecError(
                 f"the HIP codec kernels need GPU tensors; got a tensor on {t.device}"
             )
@@ -335,7 +335,16 @@ def require_slot_state(history: torch.Tensor | None, slot_index: torch.Tensor | 
         raise ValueError(f"{what}: slot_parity must be contiguous int64 with an entry per slot")
 
 
+# The current stream's handle without building a torch.cuda.Stream: 0.2 us of host time a launch
+# instead of 2.1 (an eager transformer layer's seven launches cost 8 - 9 us each on the host, more
+# than most of their kernels take). None where torch is built without a GPU backend.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_handle(device: torch.device | None = None) -> int:
+    if _raw_stream is not None and type(device) is torch.device and device.type == "cuda" \
+            and device.index is not None:
+        return _raw_stream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
 
 
