@@ -12,24 +12,28 @@
 // (sglang_omni/models/qwen3_omni/components/), so the elementwise passes after each GEMM run in
 // its epilogue on the float32 accumulators.
 //
-// Workgroup: 4 waves (2 x 2) over a tile of BM rows x BN columns, each wave TM x TN MFMA tiles of
-// 16 x 16 (v_mfma_f32_16x16x32_bf16). K runs in stages of 64: the stage's A rows and W rows travel
-// by LDS DMA (buffer_load ... lds, 16 bytes a lane) into a ring of S stages, S - 1 of them in
-// flight while one is multiplied, with one barrier per stage. An LDS row is 64 bf16 (8 slots of 16
+// Workgroup: WM x WN waves over a tile of BM rows x BN columns, each wave TM x TN MFMA tiles of
+// 16 x 16 (v_mfma_f32_16x16x32_bf16). K runs in blocks of 64, G of them to a stage: the stage's A
+// rows and W rows travel by LDS DMA (buffer_load ... lds, 16 bytes a lane) into a ring of S stages,
+// S - 1 of them in flight while one is multiplied, with one barrier per stage (G = 1 where many
+// workgroups hide each other's barriers, 2 and 4 where a few rows leave one workgroup to a CU and
+// the chain of barriers is the time). An LDS row is 64 bf16 (8 slots of 16
 // bytes), slot s of row r stored at s ^ (r % 8), so the operand reads of 16 rows spread over all
 // banks; each DMA lane loads the global piece that belongs in its slot.
 //
-// Every output element accumulates its K products in one fixed order (stage by stage, the two
-// 32-wide MFMA steps of a stage in order) whatever the tile or the row count, so a row's result
+// Every output element accumulates its K products in one fixed order (block by block, the two
+// 32-wide MFMA steps of a block in order) whatever the tile or the row count, so a row's result
 // does not depend on the rows it is batched with: a chunked decode and the whole decode give the
 // same bits.
+#include <type_traits>
+
 #include "common.h"
 #include "omni_codec.h"
 #include "rope.h"
 
 namespace {
 
-constexpr int kBK = 64;         // K per stage
+constexpr int kBK = 64;         // K per block
 constexpr int kRowSlots = 8;    // 16-byte slots per staged row
 
 struct GemmParams {
@@ -70,19 +74,20 @@ OMNI_DEVICE uint32_t pack_bf16x2(float a, float b) {
 OMNI_DEVICE float silu(float g) { return g / (1.f + __expf(-g)); }
 OMNI_DEVICE float gelu_erf(float x) { return 0.5f * x * (1.f + erff(x * 0.70710678118654752f)); }
 
-template <int WM, int WN, int TM, int TN, int S>
+template <int WM, int WN, int TM, int TN, int S, int G = 1>
 struct GemmTile {
   static constexpr int NW = WM * WN;  // waves: WM down the rows, WN across the columns
   static constexpr int BM = WM * TM * 16;
   static constexpr int BN = WN * TN * 16;
   static constexpr int A_ELEMS = BM * kBK;
   static constexpr int B_ELEMS = BN * kBK;
-  static constexpr int STAGE = A_ELEMS + B_ELEMS;  // bf16 elements
+  static constexpr int BLOCK = A_ELEMS + B_ELEMS;  // bf16 elements of one K block
+  static constexpr int STAGE = G * BLOCK;
   static constexpr size_t lds_bytes() { return (size_t)S * STAGE * 2; }
   // 64-lane DMA instructions of a stage (each fills 8 staged rows), shared by the waves
   static constexpr int A_PER_WAVE = BM * kRowSlots / 64 / NW;
   static constexpr int B_PER_WAVE = BN * kRowSlots / 64 / NW;
-  static constexpr int PER_WAVE = A_PER_WAVE + B_PER_WAVE;
+  static constexpr int PER_WAVE = G * (A_PER_WAVE + B_PER_WAVE);
   static_assert((BM * kRowSlots / 64) % NW == 0 && (BN * kRowSlots / 64) % NW == 0, "DMA split");
 };
 
@@ -199,9 +204,19 @@ OMNI_DEVICE void rope_kv_epilogue(const GemmParams& p, const f32x4 (&acc)[TM][4]
   }
 }
 
-template <int WM, int WN, int TM, int TN, int S, bool ROPE = false>
+// multiply() of the stages from kt on, the last LATER + 1 of K: one stage less in flight behind
+// each.
+template <int LATER, class F>
+OMNI_DEVICE void multiply_tail(int stages, int kt, F& multiply) {
+  if constexpr (LATER >= 0) {
+    if (stages > LATER) multiply(kt++, std::integral_constant<int, LATER>{});
+    multiply_tail<LATER - 1>(stages, kt, multiply);
+  }
+}
+
+template <int WM, int WN, int TM, int TN, int S, int G, bool ROPE = false>
 __global__ void __launch_bounds__(64 * WM * WN) gemm_kernel(const GemmParams p) {
-  using T = GemmTile<WM, WN, TM, TN, S>;
+  using T = GemmTile<WM, WN, TM, TN, S, G>;
   static_assert(!ROPE || TN == 4, "the rotary epilogue takes one 64-column head per wave");
   extern __shared__ __attribute__((aligned(16))) u16 lds[];
   const int tid = threadIdx.x;
@@ -238,21 +253,24 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_kernel(const GemmParams p) 
       b_off[i] = n0 + row < p.n ? (uint32_t)((n0 + row) * p.k + slot * 8) * 2u : kOutOfRange;
     }
   }
-  const int stages = p.k / kBK;
+  const int stages = p.k / (G * kBK);
   auto issue = [&](int kt) __attribute__((always_inline)) {
-    u16* st = lds + (kt % S) * T::STAGE;
-    const int kb = kt * kBK * 2;
 #pragma unroll
-    for (int i = 0; i < T::A_PER_WAVE; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          ar, (__attribute__((address_space(3))) void*)(st + (wave * T::A_PER_WAVE + i) * 512), 16,
-          (int)a_off[i], kb, 0, 0);
+    for (int g = 0; g < G; ++g) {
+      u16* st = lds + (kt % S) * T::STAGE + g * T::BLOCK;
+      const int kb = (kt * G + g) * kBK * 2;
 #pragma unroll
-    for (int i = 0; i < T::B_PER_WAVE; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          wr, (__attribute__((address_space(3))) void*)(st + T::A_ELEMS +
-                                                        (wave * T::B_PER_WAVE + i) * 512),
-          16, (int)b_off[i], kb, 0, 0);
+      for (int i = 0; i < T::A_PER_WAVE; ++i)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            ar, (__attribute__((address_space(3))) void*)(st + (wave * T::A_PER_WAVE + i) * 512), 16,
+            (int)a_off[i], kb, 0, 0);
+#pragma unroll
+      for (int i = 0; i < T::B_PER_WAVE; ++i)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            wr, (__attribute__((address_space(3))) void*)(st + T::A_ELEMS +
+                                                          (wave * T::B_PER_WAVE + i) * 512),
+            16, (int)b_off[i], kb, 0, 0);
+    }
   };
 
   // operand reads: row r (a multiple of 16 plus lane % 16) of the A or W region, logical slot
@@ -276,21 +294,20 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_kernel(const GemmParams p) 
   for (int kt = 0; kt < S - 1; ++kt)
     if (kt < stages) issue(kt);
   if constexpr (ROPE) rope_rows_positions<TM>(p, m0 + wm * TM * 16, lane, rope);
-  for (int kt = 0; kt < stages; ++kt) {
-    // this wave's DMA of stage kt is complete once at most the later stages' instructions are
-    // outstanding; then every wave's (the barrier), which also ends every read of the buffer that
-    // stage kt + S - 1 refills
-    if (kt + S - 2 < stages) {
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 2) * T::PER_WAVE) : "memory");
-    } else {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
+  // one stage, LATER stages in flight behind it: this wave's DMA of stage kt is complete once at
+  // most the later stages' instructions are outstanding; then every wave's (the barrier), which
+  // also ends every read of the buffer that stage kt + S - 1 refills
+  auto multiply = [&](int kt, auto later) __attribute__((always_inline)) {
+    constexpr int LATER = decltype(later)::value;
+    static_assert(LATER * T::PER_WAVE <= 63, "vmcnt range");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LATER * T::PER_WAVE) : "memory");
     asm volatile("s_barrier" ::: "memory");
-    if (kt + S - 1 < stages) issue(kt + S - 1);
+    if constexpr (LATER == S - 2)
+      if (kt + S - 1 < stages) issue(kt + S - 1);
     const u16* st = lds + (kt % S) * T::STAGE;
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int rd = s ? rd1 : rd0;
+    for (int s = 0; s < 2 * G; ++s) {
+      const int rd = (s / 2) * T::BLOCK + (s % 2 ? rd1 : rd0);
       bf16x8 av[TM], bv[TN];
 #pragma unroll
       for (int i = 0; i < TM; ++i)
@@ -304,7 +321,11 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_kernel(const GemmParams p) 
         for (int j = 0; j < TN; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bv[j], av[i], acc[i][j], 0, 0, 0);
     }
-  }
+  };
+  int kt = 0;
+  for (; kt + S - 2 < stages; ++kt) multiply(kt, std::integral_constant<int, S - 2>{});
+  // the last S - 2 stages (all of them, if K has fewer), each with one stage less behind it
+  multiply_tail<S - 3>(stages, kt, multiply);
 
   // epilogue: lane holds row m0 + wm TM 16 + 16 i + lane % 16, columns n0 + wn TN 16 + 16 j +
   // 4 (lane / 16) .. + 3 of tile (i, j)
@@ -377,12 +398,13 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_kernel(const GemmParams p) 
   }
 }
 
-template <int WM, int WN, int TM, int TN, int S, bool ROPE = false>
+template <int WM, int WN, int TM, int TN, int S, bool ROPE = false, int G = 1>
 int launch(GemmParams p, hipStream_t stream) {
-  using T = GemmTile<WM, WN, TM, TN, S>;
+  using T = GemmTile<WM, WN, TM, TN, S, G>;
+  if (p.k % (G * kBK) != 0) return OMNI_ERR_UNSUPPORTED;
   p.row_tiles = (p.rows + T::BM - 1) / T::BM;
   p.col_tiles = (p.n + T::BN - 1) / T::BN;
-  auto k = gemm_kernel<WM, WN, TM, TN, S, ROPE>;
+  auto k = gemm_kernel<WM, WN, TM, TN, S, G, ROPE>;
   static const bool raised = [&] {
     return hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)T::lds_bytes()) == hipSuccess;
@@ -492,9 +514,31 @@ extern "C" int omni_gemm(const omni_gemm_args* a, omni_stream_t stream) {
   // wave per SIMD hides the stage barrier and the LDS latency the one-wave tiles wait on (qkv
   // 768 x 1024 -> 3072 14.4 -> 13.1 us, down 768 x 3072 -> 1024 17.8 -> 16.5 us); deeper rings
   // and 128 x 128 tiles were slower.
+  //
+  // Few rows: the tiles above leave most CUs idle while each workgroup walks K alone, one
+  // barrier and one LDS round trip (~0.28 us) per 64 of K, and a deeper ring does not help: the
+  // data is there, the chain is what costs. So the smallest tile that still gives each workgroup
+  // a CU of its own, and K in stages of 256 (128): four (two) K blocks of the same layout per
+  // barrier, whose LDS reads and MFMAs overlap. us at rows x K -> columns, before and after:
+  //   16 x 32, 2 waves, 4 stages of 256, 96 KiB: 80 x 1024 -> 1024 6.4 -> 3.4, 80 x 3072 ->
+  //     1024 13.7 -> 6.2, 16 x 1024 -> 4096 6.8 -> 4.3
+  //   32 x 32, 4 waves, 4 stages of 256, 128 KiB: 160 x 3072 -> 1024 13.6 -> 7.1 (16 x 32 at two
+  //     rounds of workgroups 10.6), 240 x 4096 -> 1024 17.1 -> 8.7
+  //   32 x 64, 4 waves, 3 stages of 128, 72 KiB: 320 x 3072 -> 1024 13.7 -> 10.7 (32 x 32 12.5),
+  //     480 x 4096 -> 1024 18.0 -> 13.7, 40 x 1024 -> 6144 gated 6.3 -> 5.4
+  // Past one workgroup a CU the larger tiles win (900 x 3072 -> 1024: 32 x 64 17.6, 64 x 64
+  // 15.1; 80 x 1024 -> 6144 gated, 288 workgroups: 7.1 and 6.9).
   int config = a->config;
   if (config == 0) {
-    if (a->n % 128 == 0 && tiles_of(a->rows, a->n, 64, 128) >= compute_units())
+    const int cus = compute_units();
+    const bool one_tile = epi != OMNI_GEMM_SILU_MUL;  // the gated epilogue takes two per wave
+    if (one_tile && a->k % 256 == 0 && tiles_of(a->rows, a->n, 16, 32) <= cus)
+      return launch<1, 2, 1, 1, 4, false, 4>(p, s);
+    if (one_tile && a->k % 256 == 0 && tiles_of(a->rows, a->n, 32, 32) <= cus)
+      return launch<2, 2, 1, 1, 4, false, 4>(p, s);
+    if (a->k % 128 == 0 && tiles_of(a->rows, a->n, 32, 64) <= cus)
+      return launch<2, 2, 1, 2, 3, false, 2>(p, s);
+    if (a->n % 128 == 0 && tiles_of(a->rows, a->n, 64, 128) >= cus)
       config = 3;
     else
       config = epi == OMNI_GEMM_SILU_MUL ? 5 : 4;
@@ -546,9 +590,19 @@ extern "C" int omni_gemm_rope_kv(const omni_gemm_args* a, int64_t frames, int64_
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   // one 64-column head per wave: 64 x 128 tiles of 4 waves (2 x 2, each 32 rows) or of 8 (4 x
   // 2, each 16 rows). At 768 x 1024 -> 3072 with rings: 15.3 and 16.1 us (the two-launch form
-  // 19.5 us; its GEMM alone 11.1 - 12.1 us, the ring writes ~2.2 us of the difference)
-  const int config = a->config == 0 ? 1 : a->config;
+  // 19.5 us; its GEMM alone 11.1 - 12.1 us, the ring writes ~2.2 us of the difference).
+  // Few rows, as in omni_gemm: one column of 1, 2 or 4 such waves per workgroup (16, 32, 64 rows
+  // x 64 columns; rings of 3, 3, 2 stages of 256: 120, 144, 128 KiB) while each gets a CU of its
+  // own: 80 x 1024 -> 3072 10.5 -> 6.9 us, 160 rows 10.6 -> 7.2, 320 rows 10.8 -> 8.1 (two
+  // rounds: 14.3 at 640 rows, where 64 x 128 takes 11.2).
   if (a->n % 128 != 0) return OMNI_ERR_UNSUPPORTED;
+  if (a->config == 0 && a->k % 256 == 0) {
+    const int cus = compute_units();
+    if (tiles_of(a->rows, a->n, 16, 64) <= cus) return launch<1, 1, 1, 4, 3, true, 4>(p, s);
+    if (tiles_of(a->rows, a->n, 32, 64) <= cus) return launch<2, 1, 1, 4, 3, true, 4>(p, s);
+    if (tiles_of(a->rows, a->n, 64, 64) <= cus) return launch<4, 1, 1, 4, 2, true, 4>(p, s);
+  }
+  const int config = a->config == 0 ? 1 : a->config;
   switch (config) {
     case 1: return launch<2, 2, 2, 4, 3, true>(p, s);
     case 6: return launch<4, 2, 1, 4, 3, true>(p, s);
