@@ -129,9 +129,7 @@ class HifiGanVocoder:
                 xj = view(xb[j], length, cout) if j < 2 else None
                 src = q
                 for m, (c1, c2) in enumerate(pairs):
-                    # (k = 11 pairs measured slower as one launch: 540-610 against 435 us for
-                    # the two launches at 16 x 240 000 samples, the tile's 2 x 30-row x halo)
-                    paired = self.pairs and c1.taps < 11 and resblock_pair_supported(c1, c2)
+                    paired = self.pairs and resblock_pair_supported(c1, c2)
                     last_m = m + 1 == len(pairs)
                     resid = xstage if m == 0 else (xj if j < 2 else xstage)
                     if not last_m:

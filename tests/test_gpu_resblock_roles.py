@@ -1,0 +1,99 @@
+"""``omni_resblock_pair`` at the edges of its tiles (256 - (k - 1) output positions, workgroups that
+take several tiles, rows of a few positions) and over the forms its epilogue takes (no bias, no
+residual, float32 output, Snake / tanh activation, strided tensors, float16 and float32 streams,
+the mix with and without the stream): the bits of the two ``omni_conv1d_fused`` launches, and
+nothing written between or past the rows."""
+
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+from sglang_omni_amd import _native as N
+from sglang_omni_amd.kernels.conv import fused_conv, pack_conv1d, resblock_pair
+
+pytestmark = pytest.mark.gpu
+
+SLOPE = 0.1
+
+
+def _pair(k, d, gpu, bias=True):
+    g = torch.Generator().manual_seed(100 * k + d)
+    def conv(dilation):
+        return pack_conv1d(torch.randn(32, 32, k, generator=g) / math.sqrt(32 * k),
+                           torch.randn(32, generator=g) * 0.1 if bias else None,
+                           dilation=dilation, causal=False).to(gpu)
+    return conv(d), conv(1)
+
+
+def _rows(batch, length, pitch, dtype, gpu, seed=None):
+    """[batch, length, 32] with rows `pitch` elements apart in a NaN buffer (or random)."""
+    buf = torch.full((batch, length + 3, pitch), float("nan"), dtype=dtype, device=gpu)
+    view = buf[:, :length, :32]
+    if seed is not None:
+        g = torch.Generator().manual_seed(seed)
+        view.copy_(torch.randn(batch, length, 32, generator=g).to(dtype))
+    return buf, view
+
+
+def _both(x, c1, c2, gpu, *, out_dtype=torch.bfloat16, stream=torch.float16, pitch=32,
+          residual=True, mix=False, sum_out=True, out=True, **kw):
+    batch, length, _ = x.shape
+    if residual:
+        kw["residual"] = _rows(batch, length, pitch, stream, gpu, 7)[1]
+    if mix:
+        kw["mix"] = (_rows(batch, length, pitch, stream, gpu, 8)[1],
+                     _rows(batch, length, pitch, stream, gpu, 9)[1], 1.0 / 3.0)
+    results = []
+    for paired in (False, True):
+        buffers = []
+        o = s = None
+        if out:
+            buf, o = _rows(batch, length, pitch, out_dtype, gpu)
+            buffers.append(buf)
+        if sum_out:
+            buf, s = _rows(batch, length, pitch, stream, gpu)
+            buffers.append(buf)
+        if paired:
+            resblock_pair(x, c1, c2, o, slope1=SLOPE, sum_out=s, **kw)
+        else:
+            h = torch.empty(batch, length, 32, dtype=torch.bfloat16, device=gpu)
+            fused_conv(x, c1, h, activation=N.ACT_LEAKY_RELU, slope=SLOPE)
+            fused_conv(h, c2, o, sum_out=s, **kw)
+        results.append(buffers)
+    for want, got in zip(*results):
+        assert not want[:, :length, :32].isnan().any()
+        bits = torch.int32 if want.dtype == torch.float32 else torch.int16
+        assert torch.equal(got.view(bits), want.view(bits))  # the NaNs around the rows too
+
+
+@pytest.mark.parametrize("k", [3, 7, 11])
+@pytest.mark.parametrize("d", [1, 2, 5])
+def test_tile_edges(gpu, k, d):
+    c1, c2 = _pair(k, d, gpu)
+    bp = 256 - (k - 1)
+    for batch, length in ((1, 1), (2, 3), (3, bp - 1), (1, bp), (2, bp + 1), (1, 2 * bp + 17),
+                          (2, 1100 * bp + 5), (700, 40)):
+        x = _rows(batch, length, 32, torch.bfloat16, gpu, 5)[1]
+        _both(x, c1, c2, gpu, activation=N.ACT_LEAKY_RELU, slope=SLOPE)
+
+
+@pytest.mark.parametrize("k", [3, 7, 11])
+@pytest.mark.parametrize("stream", [torch.float16, torch.float32])
+def test_epilogue_forms(gpu, k, stream):
+    c1, c2 = _pair(k, 3, gpu)
+    plain1, plain2 = _pair(k, 3, gpu, bias=False)
+    a = torch.rand(32, device=gpu) + 0.5
+    x = _rows(2, 777, 48, torch.bfloat16, gpu, 6)[1]  # strided rows
+    lrelu = dict(activation=N.ACT_LEAKY_RELU, slope=0.01)
+    for pitch in (32, 40):
+        kw = dict(stream=stream, pitch=pitch)
+        _both(x, plain1, plain2, gpu, residual=False, sum_out=False, **kw)
+        _both(x, c1, c2, gpu, residual=False, **kw, **lrelu)
+        _both(x, c1, c2, gpu, out=False, **kw)
+        _both(x, c1, c2, gpu, mix=True, sum_out=False, **kw, **lrelu)
+        _both(x, c1, c2, gpu, mix=True, **kw)
+        _both(x, c1, c2, gpu, out_dtype=torch.float32, activation=N.ACT_TANH, **kw)
+        _both(x, c1, c2, gpu, activation=N.ACT_SNAKE, act_a=a, act_b=1 / a, **kw)
