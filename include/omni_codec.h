@@ -225,6 +225,9 @@ int omni_conv1d_fused(const omni_conv_args* args, omni_stream_t stream);
  *                                (c_in a multiple of 96 for taps 1 and 2); the weight2 form at
  *                                192 columns: 1. Taken for calls that leave the GPU mostly idle on
  *                                the other families' tiles, with the same bits
+ *   OMNI_CONV_KERNEL_DMA_MID     LDS-DMA staged as OMNI_CONV_KERNEL_DMA with smaller tiles (bf16
+ *                                weights, taps 1, 2 or 7, no weight2): 3 each, with the same bits;
+ *                                taken where that list's tiles fill the GPU badly
  * omni_conv1d_fused_with runs the same arithmetic with the family and the list's config-th entry
  * (1-based) named by the caller (OMNI_ERR_UNSUPPORTED when they cannot serve the call); the
  * results of every configuration agree to float32 summation order. omni_conv1d_plan reports,
@@ -240,7 +243,8 @@ enum {
   OMNI_CONV_KERNEL_STAGED = 2,
   OMNI_CONV_KERNEL_STAGED11 = 3,
   OMNI_CONV_KERNEL_FUSED_UNIT = 4,
-  OMNI_CONV_KERNEL_SMALL = 5
+  OMNI_CONV_KERNEL_SMALL = 5,
+  OMNI_CONV_KERNEL_DMA_MID = 6
 };
 
 int omni_conv1d_fused_with(const omni_conv_args* args, int kernel, int config,

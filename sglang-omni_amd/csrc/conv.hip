@@ -16,29 +16,34 @@ static __device__ __align__(256) float scratch[kScratchBytes / 4];
 namespace omni_conv {
 namespace {
 
-// The time in us of the LDS-DMA tile that a bf16 call would take, as far as the small-call kernel
-// may be the faster one: a chain of staged chunks per workgroup (measured, 8 to 64 workgroups: k = 7
-// 60 us or 43 by tile at 24 chunks, 25 at 12, 16 at 6; two taps 29.5 / 18 / 14.5 at 48 / 24 / 12;
-// k = 1 12.7 / 10.9 / 9.1 at 24 / 12 / 6; the 192-channel unit 36), in rounds of 256 workgroups.
-// 0 where no such tile fits, and for narrow layers and two-tap layers of three stages, whose
-// chains are short (192 -> 576 columns at 1 280 positions: 11.0 us against 8.4).
-double large_tile_us(const ConvParams& p, bool fuse2, hipStream_t stream) {
+// The LDS-DMA tile that a bf16 call would take, where smaller tiles or the small-call kernel may be
+// the faster ones: its time in us (0 where no tile of the large lists fits, and for narrow layers
+// and two-tap layers of three stages, whose chains are short: 192 -> 576 columns at 1 280
+// positions: 11.0 us on the small kernel, 8.4 here), and whether it is one of the smaller tiles.
+struct LargeTile {
+  double us = 0;
+  bool mid = false;
+};
+LargeTile large_tile(const ConvParams& p, bool fuse2, hipStream_t stream) {
   const int chunks = p.c_in / kChunk;
-  if (p.n_cols < 192 || (p.taps == 2 && chunks <= 6)) return 0;
-  Choice ch;
-  ch.launch = false;
-  int status = OMNI_ERR_UNSUPPORTED;
+  if (p.n_cols < 192 || (p.taps == 2 && chunks <= 6)) return {};
+  Choice ch, mid;
+  ch.launch = mid.launch = false;
+  int status = OMNI_ERR_UNSUPPORTED, mid_status = OMNI_ERR_UNSUPPORTED;
   if (fuse2) status = launch_fused<false>(p, IN_RAW, ch, stream);
   else if (p.taps == 7) status = launch_dma_taps7(p, false, ch, stream);
   else if (p.taps == 2) status = launch_dma_taps2(p, false, ch, stream);
   else if (p.taps == 1) status = launch_dma_taps1(p, false, ch, stream);
-  if (status != OMNI_OK) return 0;
+  if (status != OMNI_OK) return {};
   const double rounds = (double)((ch.workgroups + 255) / 256);
-  if (fuse2) return 36 * rounds;
-  if (p.taps == 7)  // a split's reduction launch takes 4.5 us
-    return 5 + 1.6 * chunks / p.k_splits * rounds + (p.k_splits > 1 ? 4.5 : 0);
-  const int per_stage = p.taps == 2 ? 2 : 3;
-  return 7 + 0.95 * ((chunks + per_stage - 1) / per_stage) * rounds;
+  if (fuse2) return {36 * rounds, false};  // the 192-channel unit, measured
+  if (p.k_splits > 1)  // a split runs the large tiles; its reduction launch takes 4.5 us
+    return {9.5 + 1.6 * chunks / p.k_splits * rounds, false};
+  if (p.taps == 7) mid_status = launch_mid_taps7(p, mid, stream);
+  else if (p.taps == 2) mid_status = launch_mid_taps2(p, mid, stream);
+  else if (p.taps == 1) mid_status = launch_mid_taps1(p, mid, stream);
+  if (mid_status == OMNI_OK && mid.us < ch.us) return {mid.us, true};
+  return {ch.us, false};
 }
 
 // The kernel family and configuration for p: OMNI_CONV_KERNEL_AUTO picks the family by the
@@ -51,10 +56,13 @@ int dispatch(const ConvParams& p, bool x_f32, bool fp8, bool fuse2, int& kernel,
   const int in_mode = x_f32 ? IN_F32 : (p.in_act != OMNI_ACT_NONE ? IN_ACT : IN_RAW);
   int want = kernel;
   auto allowed = [&](int family) { return want == OMNI_CONV_KERNEL_AUTO || want == family; };
-  if (allowed(OMNI_CONV_KERNEL_SMALL) && in_mode == IN_RAW && !fp8 && p.c_in % kChunk == 0) {
+  const bool plain = in_mode == IN_RAW && !fp8 && p.c_in % kChunk == 0;
+  LargeTile large;
+  if (want == OMNI_CONV_KERNEL_AUTO && plain) large = large_tile(p, fuse2, stream);
+  if (allowed(OMNI_CONV_KERNEL_SMALL) && plain) {
     // a forced entry runs as asked; else the small-call kernel where it beats the tile the call
     // would take (and only where there is one: what those refuse stays refused)
-    const double than = want == OMNI_CONV_KERNEL_SMALL ? 0 : large_tile_us(p, fuse2, stream);
+    const double than = large.us;
     int status = OMNI_ERR_UNSUPPORTED;
     if (fuse2) status = launch_small_unit(p, than, ch, stream);
     else if (p.taps == 7) status = launch_small_taps7(p, than, ch, stream);
@@ -66,6 +74,14 @@ int dispatch(const ConvParams& p, bool x_f32, bool fp8, bool fuse2, int& kernel,
     }
   }
   if (want == OMNI_CONV_KERNEL_SMALL) return OMNI_ERR_UNSUPPORTED;
+  if (want == OMNI_CONV_KERNEL_DMA_MID || large.mid) {
+    kernel = OMNI_CONV_KERNEL_DMA_MID;
+    if (!plain || fuse2 || p.k_splits > 1) return OMNI_ERR_UNSUPPORTED;
+    if (p.taps == 7) return launch_mid_taps7(p, ch, stream);
+    if (p.taps == 2) return launch_mid_taps2(p, ch, stream);
+    if (p.taps == 1) return launch_mid_taps1(p, ch, stream);
+    return OMNI_ERR_UNSUPPORTED;
+  }
   // of the other families only the LDS-DMA tiles write split-K partials: a split call no DMA tile
   // fits is refused, never handed to a family that would write the whole conv into out and leave
   // the reduction summing partials nobody wrote
@@ -339,7 +355,7 @@ int conv_entry(const omni_conv_args* a, int kernel, int config, bool launch, int
                int* config_out, int* count_out, int64_t* workgroups_out, omni_stream_t stream,
                int64_t k_splits = 1, float* workspace = nullptr, int64_t workspace_bytes = 0) {
   using namespace omni_conv;
-  if (kernel < OMNI_CONV_KERNEL_AUTO || kernel > OMNI_CONV_KERNEL_SMALL || config < 0 ||
+  if (kernel < OMNI_CONV_KERNEL_AUTO || kernel > OMNI_CONV_KERNEL_DMA_MID || config < 0 ||
       (kernel == OMNI_CONV_KERNEL_AUTO && config != 0) || k_splits < 1)
     return OMNI_ERR_INVALID_ARG;
   ConvParams p;

@@ -459,12 +459,44 @@ int launch_first_fit(const ConvParams& p, Choice& ch, hipStream_t stream) {
   return choose_and_launch(ch, n, fits, wgs, launch, pick, p, stream);
 }
 
+// A tile's measured time on one CU, us: `fixed` + `chunk` per 32-channel chunk of c_in.
+struct TileCost {
+  double fixed, chunk;
+};
+
+// Launch the fitting configuration of the least time: its cost times the rounds its workgroups
+// take at one per CU (256). A list ordered by size and searched for the first with 256 workgroups
+// ran into rounds that are nearly empty: 768 -> 768 columns, k = 7, at 8 000 positions took 336
+// workgroups of 96 x 192 in two rounds, 90 us, where 168 of 96 x 384 take 69 in one. The costs are
+// fitted to the decoder's layers at 96 to 512 000 positions; the estimates lie within 15 % there.
+template <typename... Cfgs>
+int launch_least(const ConvParams& p, const TileCost (&cost)[sizeof...(Cfgs)], Choice& ch,
+                 hipStream_t stream) {
+  constexpr int n = sizeof...(Cfgs);
+  const bool fits[n] = {Cfgs::fits(p)...};
+  const int64_t wgs[n] = {Cfgs::workgroups(p)...};
+  int (*const launch[n])(ConvParams, hipStream_t) = {&Cfgs::launch...};
+  int pick = -1;
+  for (int i = 0; i < n; ++i) {
+    if (!fits[i]) continue;
+    const double us = (double)((wgs[i] + 255) / 256) *
+                      (cost[i].fixed + cost[i].chunk * (p.c_in / kChunk));
+    if (pick < 0 || us < ch.us) pick = i, ch.us = us;
+  }
+  return choose_and_launch(ch, n, fits, wgs, launch, pick, p, stream);
+}
+
 // Launchers by tap count (1: k = 1 convs, 2: transposed convs of kernel 2 * stride, 7: k = 7
 // convs; 3 and 11: narrow layers' k = 3 and k = 11 convs), one translation unit each.
 // `fp8`: the packed weights are E4M3 (one byte per weight, per-column scales in the epilogue).
 int launch_dma_taps1(const ConvParams& p, bool fp8, Choice& ch, hipStream_t stream);
 int launch_dma_taps2(const ConvParams& p, bool fp8, Choice& ch, hipStream_t stream);
 int launch_dma_taps7(const ConvParams& p, bool fp8, Choice& ch, hipStream_t stream);
+// The smaller tiles of the same three tap counts (bf16 weights): 96 columns x 64, 128 or 256
+// positions, for calls whose workgroups of the lists above fill the CUs badly
+int launch_mid_taps1(const ConvParams& p, Choice& ch, hipStream_t stream);
+int launch_mid_taps2(const ConvParams& p, Choice& ch, hipStream_t stream);
+int launch_mid_taps7(const ConvParams& p, Choice& ch, hipStream_t stream);
 // HiFiGAN's layers only (bf16 weights; n_cols <= 64, or a multiple of 128 or 96 for k = 3, or 128
 // for k = 11): k = 3 and k = 11
 int launch_dma_taps3(const ConvParams& p, bool fp8, Choice& ch, hipStream_t stream);

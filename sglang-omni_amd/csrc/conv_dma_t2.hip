@@ -14,10 +14,13 @@ int launch_dma_taps2(const ConvParams& p, bool fp8, Choice& ch, hipStream_t stre
                             DmaConfig<2, 4, 6, 3, 224, 2, 1, true>,
                             DmaConfig<2, 4, 3, 3, 224, 2, 2, true>,
                             DmaConfig<1, 8, 6, 3, 432, 2, 1, true>>(p, ch, stream);
-  return launch_first_fit<DmaConfig<4, 4, 3, 3, 224, 2, 1>,
-                            DmaConfig<2, 4, 6, 3, 224, 2, 1>,
-                            DmaConfig<2, 4, 3, 3, 224, 2, 2>,
-                            DmaConfig<1, 8, 6, 3, 432, 2, 1>>(p, ch, stream);
+  // (measured in one round, us at 48 / 24 / 12 chunks: 55 / 34 / 24, 59 / 37 / 25, 40 - 43 / 25 -
+  // 27 / 15, 58 / 36 / 25)
+  return launch_least<DmaConfig<4, 4, 3, 3, 224, 2, 1>,
+                      DmaConfig<2, 4, 6, 3, 224, 2, 1>,
+                      DmaConfig<2, 4, 3, 3, 224, 2, 2>,
+                      DmaConfig<1, 8, 6, 3, 432, 2, 1>>(
+      p, {{11, 0.95}, {12, 1.0}, {6.5, 0.77}, {12, 0.95}}, ch, stream);
 }
 
 }  // namespace omni_conv

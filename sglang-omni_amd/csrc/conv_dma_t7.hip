@@ -30,10 +30,12 @@ int launch_dma_taps7(const ConvParams& p, bool fp8, Choice& ch, hipStream_t stre
   if (p.k_splits > 1)  // split-K (bf16 weights): K slices of the 96 x 192 tiles (8 / 4 waves)
     return launch_first_fit<DmaConfig<2, 4, 3, 3, 368, 7, 1, false, true>,
                             DmaConfig<1, 4, 6, 3, 368, 7, 1, false, true>>(p, ch, stream);
-  return launch_first_fit<DmaConfig<2, 8, 3, 3, 496, 7, 1>,
-                            DmaConfig<1, 8, 6, 3, 496, 7, 1>,
-                            DmaConfig<2, 4, 3, 3, 368, 7, 1>,
-                            DmaConfig<1, 4, 6, 3, 368, 7, 1>>(p, ch, stream);
+  // (measured in one round, us at 24 / 12 chunks: 66.5 / 39, 70 / 41, 46 / 27, 50 / 31)
+  return launch_least<DmaConfig<2, 8, 3, 3, 496, 7, 1>,
+                      DmaConfig<1, 8, 6, 3, 496, 7, 1>,
+                      DmaConfig<2, 4, 3, 3, 368, 7, 1>,
+                      DmaConfig<1, 4, 6, 3, 368, 7, 1>>(
+      p, {{11.5, 2.3}, {11, 2.5}, {9, 1.6}, {12, 1.65}}, ch, stream);
 }
 
 }  // namespace omni_conv

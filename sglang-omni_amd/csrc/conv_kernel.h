@@ -831,6 +831,7 @@ struct Choice {
   int chosen = 0;           // 1-based entry of the list (out)
   int count = 0;            // entries in the list (out)
   int64_t workgroups = 0;   // of the chosen entry (out)
+  double us = 0;            // the chosen entry's estimated time, where the list has costs (out)
 };
 
 // Record the choice (the forced entry when one is asked for) and launch it unless the caller

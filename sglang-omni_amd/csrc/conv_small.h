@@ -439,15 +439,13 @@ struct SmallConfig {
   }
   // The launch's time in us, fitted to measurements over the decoder's layers (1 x 4 to 32 x 12
   // frames; within 25 %): what a workgroup reads at 80 KB per us, its steps' instructions, its
-  // epilogue, in rounds of one workgroup per CU, or shared evenly where a CU's LDS holds several.
+  // epilogue, times the workgroups of the fullest CU (also where its LDS holds several at once: 288
+  // of 4 waves at 768 -> 3072 columns, two taps, 96 positions take 19.6 us, 192 of 2 waves 12.1).
   static double microseconds(const ConvParams& p) {
     const double rows = (double)rows_needed(p), steps = (double)(p.c_in / kChunk) * TAPS;
     const double us = (steps * Tile::BCO * Tile::ES + rows * p.c_in * 2) / 80e3 +
                       TP * (0.018 * steps + 0.4);
-    const double rounds = workgroups(p) / 256.0;
-    const double lds = ((int64_t)(rows + 15) / 16 * 16) * (double)slab_chunks(p) * kChunk * 2;
-    const double shared = rounds > 1 ? rounds : 1;
-    return 3 + us * (lds * 2 <= 160 * 1024 ? shared : (double)((workgroups(p) + 255) / 256));
+    return 3 + us * (double)((workgroups(p) + 255) / 256);
   }
   static int launch(ConvParams p, hipStream_t stream) {
     const int64_t positions = (int64_t)p.batch * p.length;

@@ -45,10 +45,10 @@ ABI_VERSION = 11
 
 # kernel families of omni_conv1d_fused (omni_conv1d_plan / omni_conv1d_fused_with)
 (CONV_KERNEL_AUTO, CONV_KERNEL_DMA, CONV_KERNEL_STAGED, CONV_KERNEL_STAGED11,
- CONV_KERNEL_FUSED_UNIT, CONV_KERNEL_SMALL) = range(6)
+ CONV_KERNEL_FUSED_UNIT, CONV_KERNEL_SMALL, CONV_KERNEL_DMA_MID) = range(7)
 CONV_KERNEL_NAMES = {CONV_KERNEL_DMA: "dma", CONV_KERNEL_STAGED: "staged",
                      CONV_KERNEL_STAGED11: "staged11", CONV_KERNEL_FUSED_UNIT: "fused_unit",
-                     CONV_KERNEL_SMALL: "small"}
+                     CONV_KERNEL_SMALL: "small", CONV_KERNEL_DMA_MID: "dma_mid"}
 
 
 class ConvArgs(ctypes.Structure):
