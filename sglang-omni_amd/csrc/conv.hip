@@ -36,7 +36,7 @@ LargeTile large_tile(const ConvParams& p, bool fuse2, hipStream_t stream) {
   else if (p.taps == 1) status = launch_dma_taps1(p, false, ch, stream);
   if (status != OMNI_OK) return {};
   const double rounds = (double)((ch.workgroups + 255) / 256);
-  if (fuse2) return {36 * rounds, false};  // the 192-channel unit, measured
+  if (fuse2) return {ch.us > 0 ? ch.us : 36 * rounds, false};  // (the 192-channel unit's tiles, measured)
   if (p.k_splits > 1)  // a split runs the large tiles; its reduction launch takes 4.5 us
     return {9.5 + 1.6 * chunks / p.k_splits * rounds, false};
   if (p.taps == 7) mid_status = launch_mid_taps7(p, mid, stream);

@@ -26,13 +26,14 @@
 
 namespace omni_conv {
 
+template <int TP_>
 struct FusedDmaTile {
-  static constexpr int WAVES_CO = 2, WAVES_P = 4, TCO = 6, TP = 3;
-  static constexpr int MAX_ROWS = 192 + 2 * kMaxHalo;
+  static constexpr int WAVES_CO = 2, WAVES_P = 4, TCO = 6, TP = TP_;
+  static constexpr int MAX_ROWS = WAVES_P * TP * 16 + 2 * kMaxHalo;
   using Base = ConvTile<WAVES_CO, WAVES_P, TCO, TP, MAX_ROWS, 7>;  // epilogue geometry
   static constexpr int NT = Base::NT;
   static constexpr int BCO = Base::BCO;  // 192: every channel
-  static constexpr int BP = Base::BP;    // 192 positions
+  static constexpr int BP = Base::BP;    // 64 TP positions
   static constexpr int NW = NT / 64;
   static constexpr int CH = BCO / kChunk;
   // 16-byte slots per weight row of a 4-tap / 3-tap stage, plus two pad slots: a pitch of 2 mod 4
@@ -52,7 +53,8 @@ struct FusedDmaTile {
   static constexpr int W2_PIECES = (NIW2 + NW - 1) / NW;
   static constexpr int H_ELEMS = CH * BP * kChunk;
   // a ring buffer: a stage, then W2 or h
-  static constexpr int BUF = XCHUNK + WSTAGE > H_ELEMS ? XCHUNK + WSTAGE : H_ELEMS;
+  static constexpr int AFTER = W2_ELEMS > H_ELEMS ? W2_ELEMS : H_ELEMS;
+  static constexpr int BUF = XCHUNK + WSTAGE > AFTER ? XCHUNK + WSTAGE : AFTER;
   static constexpr size_t ring_bytes = 2 * (size_t)BUF * 2;
   static constexpr size_t epi_bytes = (size_t)Base::EPI_ROWS * Base::EPITCH * 4;
   static constexpr size_t coef_offset = ring_bytes > epi_bytes ? ring_bytes : epi_bytes;
@@ -65,9 +67,10 @@ struct FusedDmaTile {
 
 // (internal linkage: the header reaches more than one translation unit, and only the bf16
 // fused launcher launches it)
+template <int TP_>
 static __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
     fused_unit_dma_kernel(const ConvParams p) {
-  using Tile = FusedDmaTile;
+  using Tile = FusedDmaTile<TP_>;
   constexpr int NT = Tile::NT;
   constexpr int NW = Tile::NW;
   constexpr int BCO = Tile::BCO;
@@ -406,8 +409,9 @@ static __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu
                                                                     wco0);
 }
 
-struct FusedDmaConfig {
-  using Tile = FusedDmaTile;
+template <int TP>
+struct FusedDmaSize {
+  using Tile = FusedDmaTile<TP>;
 
   // Staged rows of the fullest tile: BP positions over at most nseg row segments, each with its
   // own halo.
@@ -418,12 +422,7 @@ struct FusedDmaConfig {
     return bp + nseg * p.halo;
   }
 
-  // A 192-channel unit (k7 conv of C_in = C_out = 192, then the k1 conv 192 -> 192) whose staged
-  // rows fit, with no mix in its epilogue (the register-staged kernels take that).
-  static bool fits(const ConvParams& p) {
-    return p.taps == 7 && p.n_cols == Tile::BCO && p.c_out == Tile::BCO && p.c_in == Tile::BCO &&
-           p.weight2 != nullptr && p.mix_a == nullptr && rows_needed(p) <= Tile::MAX_ROWS;
-  }
+  static bool fits(const ConvParams& p) { return rows_needed(p) <= Tile::MAX_ROWS; }
 
   static int64_t workgroups(const ConvParams& p) {
     return ((int64_t)p.batch * p.length + Tile::BP - 1) / Tile::BP;
@@ -432,12 +431,61 @@ struct FusedDmaConfig {
   static int launch(ConvParams p, hipStream_t stream) {
     p.p_tiles = (int)workgroups(p);
     p.n_tiles = 1;
-    auto k = fused_unit_dma_kernel;
+    auto k = fused_unit_dma_kernel<TP>;
     static const bool raised = raise_lds_limit((const void*)k);
     (void)raised;
     hipLaunchKernelGGL(k, dim3((unsigned)p.p_tiles), dim3(Tile::NT), Tile::lds_bytes, stream, p);
     OMNI_LAUNCH_CHECK();
     return OMNI_OK;
+  }
+};
+
+struct FusedDmaConfig {
+  // A 192-channel unit (k7 conv of C_in = C_out = 192, then the k1 conv 192 -> 192) whose staged
+  // rows fit, with no mix in its epilogue (the register-staged kernels take that).
+  static bool fits(const ConvParams& p) {
+    return p.taps == 7 && p.n_cols == 192 && p.c_out == 192 && p.c_in == 192 &&
+           p.weight2 != nullptr && p.mix_a == nullptr && FusedDmaSize<3>::fits(p);
+  }
+
+  // The tile of 64 TP positions: the least time at one workgroup per CU, its measured time (21, 29
+  // and 37 us; the weight stages, which are the same for each, keep it from shrinking with the
+  // tile) times its rounds. us at TP = 1 / 2 / 3: 15 360 positions 24 / 30 / 37, 30 720 44 / 32 /
+  // 39, 60 036 82 / 58 / 73 (313 tiles of 192 in two rounds, the second a fifth full), 80 000
+  // 103 / 84 / 74, 245 760 315 / 235 / 199.
+  static constexpr double kUs[3] = {21, 29, 37};
+  static int tp(const ConvParams& p, double* us) {
+    const int64_t wgs[3] = {FusedDmaSize<1>::workgroups(p), FusedDmaSize<2>::workgroups(p),
+                            FusedDmaSize<3>::workgroups(p)};
+    const bool fit[3] = {FusedDmaSize<1>::fits(p), FusedDmaSize<2>::fits(p), true};
+    int pick = 3;
+    *us = (double)((wgs[2] + 255) / 256) * kUs[2];
+    for (int t = 2; t >= 1; --t) {
+      const double at = (double)((wgs[t - 1] + 255) / 256) * kUs[t - 1];
+      if (fit[t - 1] && at < *us) pick = t, *us = at;
+    }
+    return pick;
+  }
+  static double microseconds(const ConvParams& p) {
+    double us;
+    tp(p, &us);
+    return us;
+  }
+  static int64_t workgroups(const ConvParams& p) {
+    double us;
+    switch (tp(p, &us)) {
+      case 1: return FusedDmaSize<1>::workgroups(p);
+      case 2: return FusedDmaSize<2>::workgroups(p);
+      default: return FusedDmaSize<3>::workgroups(p);
+    }
+  }
+  static int launch(ConvParams p, hipStream_t stream) {
+    double us;
+    switch (tp(p, &us)) {
+      case 1: return FusedDmaSize<1>::launch(p, stream);
+      case 2: return FusedDmaSize<2>::launch(p, stream);
+      default: return FusedDmaSize<3>::launch(p, stream);
+    }
   }
 };
 
@@ -457,6 +505,7 @@ int launch_fused_list(const ConvParams& p, int in_mode, Choice& ch, hipStream_t 
     dma_fits = in_mode == IN_RAW && Dma::fits(p);
     dma_wgs = Dma::workgroups(p);
     dma_run = &Dma::launch;
+    if (dma_fits) ch.us = Dma::microseconds(p);
   }
   const bool fits[3] = {dma_fits, Full::fits(p, true), Short::fits(p, true)};
   const int64_t wgs[3] = {dma_wgs, Full::workgroups(p), Short::workgroups(p)};
