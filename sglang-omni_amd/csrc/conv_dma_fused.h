@@ -26,6 +26,15 @@
 
 namespace omni_conv {
 
+// f(0) .. f(N - 1), each index a compile-time constant.
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void static_for(const F& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<N, I + 1>(f);
+  }
+}
+
 template <int TP_>
 struct FusedDmaTile {
   static constexpr int WAVES_CO = 2, WAVES_P = 4, TCO = 6, TP = TP_;
@@ -210,57 +219,55 @@ static __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu
   // Stage s: chunk kc = s / 2, taps 0-3 (s even) or 4-6 (s odd): the taps' weights into ring
   // buffer s % 2 and, for the chunk's first stage, its input rows into buffer kc % 2 (where both
   // of the chunk's stages read them: the other chunk's rows there were last read two stages back).
-  auto issue = [&](int s) __attribute__((always_inline)) {
-    const int kc = s >> 1;
-    const int g = s & 1;
+  // A stage's DMA is a list of this wave's instructions (weights, then input rows); issue() sends
+  // the part [from, to) of it.
+  auto issue = [&](int kc, auto gc, auto from_c, auto to_c) __attribute__((always_inline)) {
+    constexpr int g = decltype(gc)::value;
+    constexpr int from = decltype(from_c)::value, to = decltype(to_c)::value;
+    constexpr int W = g == 0 ? Tile::W4_PIECES : Tile::W3_PIECES;
+    constexpr int NIW = g == 0 ? Tile::NIW4 : Tile::NIW3;
     u16* xs = buf_of(kc & 1);
-    u16* ws = buf_of(s & 1) + Tile::XCHUNK;
+    u16* ws = buf_of(g) + Tile::XCHUNK;
     const uint32_t wbase = (uint32_t)((kc * p.n_cols * 7 + g * 4) * kChunk * 2);
-    if (g == 0) {
 #pragma unroll
-      for (int u = 0; u < Tile::W4_PIECES; ++u) {
-        const int iw = wave + u * NW;
-        if (iw < Tile::NIW4)
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, (lds_ptr_t)(ws + iw * 64 * 8), 16,
-                                                   (int)woff4[u], (int)wbase, 0, 0);
-      }
-    } else {
-#pragma unroll
-      for (int u = 0; u < Tile::W3_PIECES; ++u) {
-        const int iw = wave + u * NW;
-        if (iw < Tile::NIW3)
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, (lds_ptr_t)(ws + iw * 64 * 8), 16,
-                                                   (int)woff3[u], (int)wbase, 0, 0);
-      }
+    for (int u = 0; u < W; ++u) {
+      const int iw = wave + u * NW;
+      if (u >= from && u < to && iw < NIW)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, (lds_ptr_t)(ws + iw * 64 * 8), 16,
+                                                 (int)(g == 0 ? woff4[u % Tile::W4_PIECES]
+                                                              : woff3[u % Tile::W3_PIECES]),
+                                                 (int)wbase, 0, 0);
     }
-    if (g != 0) return;
-    const uint32_t xbase = (uint32_t)(kc * kChunk * 2);
+    if constexpr (g == 0) {
+      const uint32_t xbase = (uint32_t)(kc * kChunk * 2);
 #pragma unroll
-    for (int u = 0; u < Tile::X_PIECES; ++u) {
-      const int ii = wave + u * NW;
-      if (ii < Tile::NIX) {
-        const unsigned mode = (xmode >> (2 * u)) & 3u;
-        lds_ptr_t dst = (lds_ptr_t)(xs + ii * 64 * 8);
-        if (mode == 1u)
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(x_rsrc, dst, 16, (int)((uint32_t)xoff[u] * 2u),
-                                                   (int)xbase, 0, 0);
-        else if (mode == 2u)  // with the non-temporal hint (aux 2), which keeps the compiler
-                              // from merging the two DMAs into one whose buffer descriptor
-                              // differs between lanes (a readfirstlane loop)
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(h_rsrc, dst, 16, (int)((uint32_t)xoff[u] * 2u),
-                                                   (int)xbase, 0, 2);
+      for (int u = 0; u < Tile::X_PIECES; ++u) {
+        const int ii = wave + u * NW;
+        if (W + u >= from && W + u < to && ii < Tile::NIX) {
+          const unsigned mode = (xmode >> (2 * u)) & 3u;
+          lds_ptr_t dst = (lds_ptr_t)(xs + ii * 64 * 8);
+          if (mode == 1u)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(x_rsrc, dst, 16, (int)((uint32_t)xoff[u] * 2u),
+                                                     (int)xbase, 0, 0);
+          else if (mode == 2u)  // with the non-temporal hint (aux 2), which keeps the compiler
+                                // from merging the two DMAs into one whose buffer descriptor
+                                // differs between lanes (a readfirstlane loop)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(h_rsrc, dst, 16, (int)((uint32_t)xoff[u] * 2u),
+                                                     (int)xbase, 0, 2);
+        }
       }
     }
   };
   // W2 ([C/32][C][32] as stored) into ring buffer b: 64-byte rows, slot s of row r holding the
   // row's piece s ^ ((r / 2) % 4)
-  auto issue_w2 = [&](int b) __attribute__((always_inline)) {
+  auto issue_w2 = [&](int b, auto from_c, auto to_c) __attribute__((always_inline)) {
+    constexpr int from = decltype(from_c)::value, to = decltype(to_c)::value;
     u16* w2s = buf_of(b);
 #pragma unroll
     for (int u = 0; u < Tile::W2_PIECES; ++u) {
       const int iw = wave + u * NW;
       const int slot = iw * 64 + lane;
-      if (iw < Tile::NIW2)
+      if (u >= from && u < to && iw < Tile::NIW2)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(w2_rsrc, (lds_ptr_t)(w2s + iw * 64 * 8), 16,
                                                  (int)((uint32_t)(slot ^ ((slot >> 3) & 3)) * 16u),
                                                  0, 0, 0);
@@ -299,50 +306,65 @@ static __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu
   }
 
   // ---- the k7 conv: 2 * CH stages, one barrier each; the next stage's DMA runs under this
-  // stage's MFMAs, and W2's under the last stage's
+  // stage's MFMAs, and W2's under the last stage's. A CU takes a DMA instruction's 1 KB in 16
+  // cycles, so the 58 - 74 KB of a stage sent at once after the barrier held every wave back
+  // 700 - 1 600 cycles of the stage's 4 000 before its first MFMA: each tap sends its share (1 280
+  // positions 21.2 -> 18.8 us, 80 000 74.5 -> 71.2, 122 880 109 -> 105, 245 760 202 -> 199).
   constexpr int STAGES = 2 * CH;
-  issue(0);
-  for (int s = 0; s < STAGES; ++s) {
+  // one stage: chunk kc, taps 4 G ..; NEXT: what it sends (0: the chunk's taps 4 - 6, 1: the next
+  // chunk's taps 0 - 3 and rows, 2: W2)
+  auto stage = [&](int kc, auto gc, auto next_c) __attribute__((always_inline)) {
+    constexpr int g = decltype(gc)::value;
+    constexpr int NEXT = decltype(next_c)::value;
+    constexpr int NTAPS = g == 0 ? 4 : 3;
+    constexpr int P8 = (g == 0 ? Tile::P4 : Tile::P3) * 8;  // u16 elements per weight row
+    constexpr int PIECES = NEXT == 0 ? Tile::W3_PIECES
+                                     : (NEXT == 1 ? Tile::W4_PIECES + Tile::X_PIECES : Tile::W2_PIECES);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (s + 1 < STAGES) issue(s + 1);
-    else issue_w2((s + 1) & 1);
-    if (p.hist != nullptr && (s & 1) == 0) write_history(s >> 1, (s >> 1) & 1);
-    const int g = s & 1;
-    const int t0 = g * 4;
-    const u16* xs = buf_of((s >> 1) & 1);         // the chunk's input rows
-    const u16* wsb = buf_of(s & 1) + Tile::XCHUNK;  // the stage's weights
+    if (g == 0 && p.hist != nullptr) write_history(kc, kc & 1);
+    const u16* xs = buf_of(kc & 1);              // the chunk's input rows
+    const u16* wsb = buf_of(g) + Tile::XCHUNK;  // the stage's weights
     // the stage's taps, software-pipelined: tap i + 1's operands are read from LDS before tap
     // i's MFMAs
-    auto stage_taps = [&](auto ntc) __attribute__((always_inline)) {
-      constexpr int NTAPS = decltype(ntc)::value;
-      constexpr int P8 = (NTAPS == 4 ? Tile::P4 : Tile::P3) * 8;  // u16 elements per weight row
-      auto load_tap = [&](int i, bf16x8 (&a)[TCO], bf16x8 (&bv)[TP]) __attribute__((always_inline)) {
-        const u16* wtap = wsb + (wco0 + lrow) * P8 + lk + i * kChunk;
+    auto load_tap = [&](int i, bf16x8 (&a)[TCO], bf16x8 (&bv)[TP]) __attribute__((always_inline)) {
+      const u16* wtap = wsb + (wco0 + lrow) * P8 + lk + i * kChunk;
+#pragma unroll
+      for (int cc = 0; cc < TCO; ++cc)
+        a[cc] = *reinterpret_cast<const bf16x8*>(wtap + cc * 16 * P8);
+      const int shift = (g * 4 + i) * dil;
+#pragma unroll
+      for (int t = 0; t < TP; ++t)
+        bv[t] = *reinterpret_cast<const bf16x8*>(xs + (xrow[t] + shift) * kChunk + lk);
+    };
+    bf16x8 a[2][TCO], bv[2][TP];
+    load_tap(0, a[0], bv[0]);
+    static_for<NTAPS>([&](auto ic) __attribute__((always_inline)) {
+      constexpr int i = decltype(ic)::value;
+      if (i + 1 < NTAPS) load_tap(i + 1, a[(i + 1) & 1], bv[(i + 1) & 1]);
+      constexpr std::integral_constant<int, PIECES * i / NTAPS> from{};
+      constexpr std::integral_constant<int, PIECES * (i + 1) / NTAPS> to{};
+      if constexpr (NEXT == 0) issue(kc, std::integral_constant<int, 1>{}, from, to);
+      else if constexpr (NEXT == 1) issue(kc + 1, std::integral_constant<int, 0>{}, from, to);
+      else issue_w2(STAGES & 1, from, to);
+#pragma unroll
+      for (int t = 0; t < TP; ++t)
 #pragma unroll
         for (int cc = 0; cc < TCO; ++cc)
-          a[cc] = *reinterpret_cast<const bf16x8*>(wtap + cc * 16 * P8);
-        const int shift = (t0 + i) * dil;
-#pragma unroll
-        for (int t = 0; t < TP; ++t)
-          bv[t] = *reinterpret_cast<const bf16x8*>(xs + (xrow[t] + shift) * kChunk + lk);
-      };
-      bf16x8 a[2][TCO], bv[2][TP];
-      load_tap(0, a[0], bv[0]);
-#pragma unroll
-      for (int i = 0; i < NTAPS; ++i) {
-        if (i + 1 < NTAPS) load_tap(i + 1, a[(i + 1) & 1], bv[(i + 1) & 1]);
-#pragma unroll
-        for (int t = 0; t < TP; ++t)
-#pragma unroll
-          for (int cc = 0; cc < TCO; ++cc)
-            acc[cc][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i & 1][cc], bv[i & 1][t],
-                                                                 acc[cc][t], 0, 0, 0);
-      }
-    };
-    if (g == 0) stage_taps(std::integral_constant<int, 4>{});
-    else stage_taps(std::integral_constant<int, 3>{});
+          acc[cc][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i & 1][cc], bv[i & 1][t],
+                                                               acc[cc][t], 0, 0, 0);
+    });
+  };
+  constexpr std::integral_constant<int, 0> c0{};
+  constexpr std::integral_constant<int, 1> c1{};
+  constexpr std::integral_constant<int, 2> c2{};
+  issue(0, c0, c0, std::integral_constant<int, Tile::W4_PIECES + Tile::X_PIECES>{});
+  for (int kc = 0; kc + 1 < CH; ++kc) {
+    stage(kc, c0, c0);
+    stage(kc, c1, c1);
   }
+  stage(CH - 1, c0, c0);
+  stage(CH - 1, c1, c2);
 
   // ---- h = mid_act(acc * scale + bias) as bf16 into ring buffer (STAGES - 1) % 2 once every
   // wave's reads of the last stage are done: [CH][BP][32], the four 16-byte slots of a 64-byte
@@ -448,12 +470,12 @@ struct FusedDmaConfig {
            p.weight2 != nullptr && p.mix_a == nullptr && FusedDmaSize<3>::fits(p);
   }
 
-  // The tile of 64 TP positions: the least time at one workgroup per CU, its measured time (21, 29
-  // and 37 us; the weight stages, which are the same for each, keep it from shrinking with the
+  // The tile of 64 TP positions: the least time at one workgroup per CU, its measured time (20, 28.5
+  // and 36 us; the weight stages, which are the same for each, keep it from shrinking with the
   // tile) times its rounds. us at TP = 1 / 2 / 3: 15 360 positions 24 / 30 / 37, 30 720 44 / 32 /
   // 39, 60 036 82 / 58 / 73 (313 tiles of 192 in two rounds, the second a fifth full), 80 000
-  // 103 / 84 / 74, 245 760 315 / 235 / 199.
-  static constexpr double kUs[3] = {21, 29, 37};
+  // 103 / 84 / 74, 245 760 315 / 235 / 199 (each with its DMA sent at the stage's start).
+  static constexpr double kUs[3] = {20, 28.5, 36};
   static int tp(const ConvParams& p, double* us) {
     const int64_t wgs[3] = {FusedDmaSize<1>::workgroups(p), FusedDmaSize<2>::workgroups(p),
                             FusedDmaSize<3>::workgroups(p)};
