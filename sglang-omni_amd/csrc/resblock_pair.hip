@@ -21,7 +21,7 @@
 //
 // us per pair at 16 x 240 000 positions, weights in LDS -> by roles (k = 11: two launches -> by
 // roles; its weights-in-LDS pair took 456): k = 3 200 -> 187, k = 7 314 -> 198, k = 11 400 - 440
-// -> 235; with the mix 334 -> 235, 507 -> 275, 490 -> 275; one row of 24 000 positions 10.4 ->
+// -> 235; with the mix 334 -> 235, 507 -> 275, 436 -> 275; one row of 24 000 positions 10.4 ->
 // 8.3, 13.2 -> 10.0, 18 -> 11.5.
 //
 // A tile is 256 h rows (16 groups of 16, 4 per wave) and so BP = 256 - (k - 1) output positions.
