@@ -502,8 +502,8 @@ int omni_snake_beta(const void* x, void* y, int dtype, int64_t batch, int64_t ch
  *   transposed  y[b, i, co] = bias[co] + sum_{j, c} W[g * C_in / groups + c, co - g * C_out /
  *               groups, j] x[b, q, g * C_in / groups + c] over q * stride + j * dilation = i +
  *               pad_left
- * with g = co / (C_out / groups) and inputs outside [0, length_in) zero. x, W and y at the given
- * element strides (W in the module's layout: [C_out, C_in / groups, k] for a conv, [C_in,
+ * with g = co / (C_out / groups), over the inputs inside [0, length_in): a tap outside the row adds
+ * nothing, whatever its weight (an infinite one too). x, W and y at the given element strides (W in the module's layout: [C_out, C_in / groups, k] for a conv, [C_in,
  * C_out / groups, k] for a transposed conv); y must not overlap x.
  */
 int omni_conv1d_general(const void* x, int dtype, int64_t batch, int64_t length_in, int64_t c_in,

@@ -290,6 +290,24 @@ __global__ void __launch_bounds__(kThreads) conv_general_mfma_kernel(const MfmaP
     }
   }
 
+  // A tap outside the row adds nothing, but the matrix cores multiply its staged zeros all the same,
+  // which an infinite or NaN weight turns into NaN: in the tiles at a row's ends an output that is
+  // not finite is summed again, without the taps outside (`again`: bit 4 TCO u + 4 c + e).
+  const int d_last = d0 + (nt - 1) * d_step;
+  const bool edge = u0 * p.u_step + min(d0, d_last) < 0 ||
+                    (min(u0 + BP, p.u_count) - 1) * p.u_step + max(d0, d_last) >= (int)g.length_in;
+  uint64_t again = 0;
+  static_assert(4 * TCO * TP <= 64, "a bit for each of a lane's outputs");
+  if (edge) {
+#pragma unroll
+    for (int u = 0; u < TP; ++u)
+#pragma unroll
+      for (int c = 0; c < TCO; ++c)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (!__builtin_isfinite(acc[c][u][e])) again |= 1ull << (4 * (TCO * u + c) + e);
+  }
+
   // lane: position lrow of a group of 16, output channels 4 lq .. 4 lq + 3 of 16
   T* y = reinterpret_cast<T*>(g.y) + (int64_t)b * g.y_sb;
   const bool vec = g.y_sc == 1 && g.y_st % 4 == 0 && g.y_sb % 4 == 0 && (group * cout_g) % 4 == 0 &&
@@ -318,6 +336,26 @@ __global__ void __launch_bounds__(kThreads) conv_general_mfma_kernel(const MfmaP
           if (n + e < cout_g) store_from_float<T>(y, o + e * g.y_sc, acc[c][u][e]);
       }
     }
+  }
+  while (again) {
+    const int bit = __builtin_ctzll(again);
+    again &= again - 1;
+    const int uu = u0 + u_wave + bit / (4 * TCO) * 16 + lrow;
+    const int n = n0 + co_wave + bit / 4 % TCO * 16 + lq * 4 + bit % 4;
+    const int64_t i = p.transposed ? (int64_t)uu * s + phase - g.pad_left : uu;
+    if (uu >= p.u_count || i < 0 || i >= g.length_out || n >= cout_g) continue;
+    float sum = g.bias ? load_as_float<T>(g.bias, group * cout_g + n) : 0.f;
+    for (int k = 0; k < nt; ++k) {
+      const int64_t pos = (int64_t)uu * p.u_step + d0 + (int64_t)k * d_step;
+      if (pos < 0 || pos >= g.length_in) continue;
+      const int64_t xo = (int64_t)b * g.x_sb + pos * g.x_st + ci0 * g.x_sc;
+      const int64_t wo = (int64_t)(p.transposed ? ci0 : group * cout_g + n) * g.w_s0 +
+                         (p.transposed ? n * g.w_s1 : 0) + (int64_t)(j0 + k * j_step) * g.w_s2;
+      const int64_t wc = p.transposed ? g.w_s0 : g.w_s1;
+      for (int c = 0; c < cin_g; ++c)
+        sum = fmaf(load_as_float<T>(g.w, wo + c * wc), load_as_float<T>(g.x, xo + c * g.x_sc), sum);
+    }
+    store_from_float<T>(y, i * g.y_st + (int64_t)(group * cout_g + n) * g.y_sc, sum);
   }
 }
 

@@ -119,3 +119,45 @@ def test_small_values_are_kept_and_infinities_stay_where_they_reach(gpu, dtype):
     bad = ~torch.isfinite(channels_last_conv_transpose1d(x, up, channels_last_weight(up),
                                                          up.bias)).all(dim=2)[0].cpu()
     assert bad.nonzero().flatten().tolist() == [300, 301, 302, 303, 480, 481, 482, 483]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("length,taps,groups,stride,dilation,pad,transposed", [
+    (300, 7, 1, 1, 3, 11, False),   # both ends of a row, inside a stage of taps
+    (129, 20, 2, 1, 1, 10, False),  # several stages of taps
+    (5, 7, 1, 1, 1, 3, False),      # every output is near an end
+    (200, 5, 1, 2, 2, 5, False),
+    (100, 11, 1, 5, 1, 3, True),
+    (40, 8, 2, 4, 3, 2, True),
+])
+def test_a_tap_outside_the_row_adds_nothing_whatever_its_weight(gpu, dtype, bad, length, taps, groups,
+                                                                 stride, dilation, pad, transposed):
+    """An infinite or NaN weight marks the outputs that its tap reaches inside the row; the others
+    are those of a zero weight in its place."""
+    x, w, b = draw(gpu, dtype, 2, length, 32, 48, taps, groups, transposed)
+    reach = (taps - 1) * dilation
+    out = ((length - 1) * stride + reach + 1 if transposed else (length + 2 * pad - reach - 1) // stride + 1)
+    kw = dict(groups=groups, stride=stride, dilation=dilation, transposed=transposed)
+    place = dict(c_out=48, pad_left=pad, length_out=out)
+    i, missed = torch.arange(out), 0
+    for tap in (0, taps // 2, taps - 1):
+        if transposed:
+            at = i + pad - tap * dilation
+            reached = (at % stride == 0) & (at >= 0) & (at < length * stride)
+        else:
+            at = i * stride + tap * dilation - pad
+            reached = (at >= 0) & (at < length)
+        zero, one = w.clone(), w.clone()
+        column = (3, 5, tap)  # output channel 5 of group 0 (transposed), output channel 3
+        zero[column], one[column] = 0.0, bad
+        channel = 5 if transposed else 3
+        want, got = _general(x, zero, b, **place, **kw), _general(x, one, b, **place, **kw)
+        reached = reached.to(gpu)
+        missed += int((~reached).sum())
+        assert not bool(torch.isfinite(got[:, reached, channel]).any())
+        got[:, reached, channel] = want[:, reached, channel]
+        check(got, x, zero, b, pad=pad, **kw)
+        got[:, :, channel] = want[:, :, channel]
+        assert torch.equal(got, want)
+    assert missed > 0  # outputs that a tap does not reach
