@@ -495,16 +495,17 @@ int omni_snake_beta(const void* x, void* y, int dtype, int64_t batch, int64_t ch
  * channels-last conv API (sglang_omni/utils/channels_last_conv.py:45-120), for what the MFMA
  * kernel does not take: any channel counts, groups, stride, dilation and zero padding, float32,
  * bf16 or f16 activations, weights and bias of that dtype, float32 accumulation in an order fixed by
- * the shapes and strides (on the matrix cores where the groups are wide enough), one rounding to
- * the dtype:
+ * the shapes and strides without the batch (on the matrix cores where the groups are wide enough and
+ * the row long enough), one rounding to the dtype:
  *   conv        y[b, i, co] = bias[co] + sum_{j, c} W[co, c, j] x[b, i * stride + j * dilation -
  *               pad_left, g * C_in / groups + c]
  *   transposed  y[b, i, co] = bias[co] + sum_{j, c} W[g * C_in / groups + c, co - g * C_out /
  *               groups, j] x[b, q, g * C_in / groups + c] over q * stride + j * dilation = i +
  *               pad_left
  * with g = co / (C_out / groups), over the inputs inside [0, length_in): a tap outside the row adds
- * nothing, whatever its weight (an infinite one too). x, W and y at the given element strides (W in the module's layout: [C_out, C_in / groups, k] for a conv, [C_in,
- * C_out / groups, k] for a transposed conv); y must not overlap x.
+ * nothing, whatever its weight (an infinite one too). x, W and y at the given element strides (W in
+ * the module's layout: [C_out, C_in / groups, k] for a conv, [C_in, C_out / groups, k] for a
+ * transposed conv); y must not overlap x.
  */
 int omni_conv1d_general(const void* x, int dtype, int64_t batch, int64_t length_in, int64_t c_in,
                         int64_t x_stride_b, int64_t x_stride_t, int64_t x_stride_c,

@@ -24,6 +24,8 @@
 // half of the time until each piece's offset was computed once and a stage added a uniform base.
 #pragma once
 
+#include <cmath>
+
 #include "conv_general.h"
 
 namespace omni_general {
@@ -60,6 +62,7 @@ struct MfmaParams {
   int u_tiles, n_tiles;
   int u_step;                // input rows between positions: a conv's stride, 1 transposed
   int group_taps;            // taps per stage
+  int s_dil_gcd, dil_inv;    // transposed: gcd(stride, dilation), 1 / (dilation / gcd) mod stride / gcd
   uint32_t x_bytes, w_bytes; // extents of one batch row of x and of the weight
 };
 
@@ -144,13 +147,11 @@ __global__ void __launch_bounds__(kThreads) conv_general_mfma_kernel(const MfmaP
   int j0 = 0, j_step = 1, d0 = -(int)g.pad_left, d_step = dil, nt = taps;
   if (p.transposed) {
     // tap j reaches phase r when j * dil = r (mod s): every j_step-th tap from j0 on
-    j0 = 0;
-    while (j0 < taps && j0 < s && (phase - (int)((int64_t)j0 * dil % s) + s) % s != 0) ++j0;
-    int a = s, c = dil % s;
-    while (c) { const int m = a % c; a = c; c = m; }  // a = gcd(s, dil)
+    const int a = p.s_dil_gcd;
     j_step = s / a;
     d_step = -(dil / a);
-    if (j0 >= s || j0 >= taps) nt = 0, j0 = 0;
+    j0 = phase / a * p.dil_inv % j_step;
+    if (phase % a != 0 || j0 >= taps) nt = 0, j0 = 0;
     else nt = (taps - 1 - j0) / j_step + 1;
     d0 = nt ? (phase - j0 * dil) / s : 0;
   }
@@ -168,7 +169,6 @@ __global__ void __launch_bounds__(kThreads) conv_general_mfma_kernel(const MfmaP
   const int chunks = (cin_g + KC - 1) / KC;
   const int gt = p.group_taps;
   const int tap_groups = nt > 0 ? (nt + gt - 1) / gt : 0;
-  const int stages = chunks * tap_groups;
 
   Piece<T, VX> xr[Tile::X_PIECES];
   Piece<T, VW> wr[Tile::W_PIECES];
@@ -201,14 +201,15 @@ __global__ void __launch_bounds__(kThreads) conv_general_mfma_kernel(const MfmaP
                                     (uint32_t)((j0 + k * j_step) * (int64_t)w_j)
                               : kOutOfRange;
   }
-  auto load_stage = [&](int st) __attribute__((always_inline)) {
-    const int c0 = st / tap_groups * KC, tg = st % tap_groups;
-    const int tap0 = tg * gt, count = min(gt, nt - tap0);
+  // stage (chunk c, tap group tg); the pieces past the rows it reads are left alone
+  auto load_stage = [&](int c, int tg) __attribute__((always_inline)) {
+    const int c0 = c * KC, tap0 = tg * gt, count = min(gt, nt - tap0);
     if (tap_groups > 1) place_rows(tap0, count);
+    const int x_pieces = stage_rows(count) * 4;
     const uint32_t xbase = (uint32_t)c0 * x_c;
 #pragma unroll
     for (int i = 0; i < Tile::X_PIECES; ++i)
-      xr[i].load(x_rsrc, xoff[i], xbase, x_c, cin_g - c0 - xq);
+      if (i * kThreads < x_pieces) xr[i].load(x_rsrc, xoff[i], xbase, x_c, cin_g - c0 - xq);
     const int pieces = count * BCO * 4;
     const uint32_t wbase = (uint32_t)c0 * w_c + (uint32_t)(tap0 * j_step) * w_j;
 #pragma unroll
@@ -221,13 +222,13 @@ __global__ void __launch_bounds__(kThreads) conv_general_mfma_kernel(const MfmaP
       }
     }
   };
-  auto store_stage = [&](int st) __attribute__((always_inline)) {
-    const int tg = st % tap_groups;
+  auto store_stage = [&](int tg) __attribute__((always_inline)) {
     const int count = min(gt, nt - tg * gt), pieces = count * BCO * 4;
+    const int x_pieces = stage_rows(count) * 4;
 #pragma unroll
     for (int i = 0; i < Tile::X_PIECES; ++i) {
       const int piece = tid + i * kThreads, row = piece >> 2;
-      if (row < kMaxRows)
+      if (piece < x_pieces)
         *reinterpret_cast<u32x4*>(xs + row * kRowBytes + (((piece ^ (row >> 1)) & 3) << 4)) =
             xr[i].packed();
     }
@@ -261,13 +262,15 @@ __global__ void __launch_bounds__(kThreads) conv_general_mfma_kernel(const MfmaP
     for (int u = 0; u < TP; ++u) acc[c][u] = v;
   }
 
-  if (stages > 0) load_stage(0);
-  for (int st = 0; st < stages; ++st) {
+  const int last_chunk = tap_groups ? chunks : 0;  // (a phase without taps has no stages)
+  if (last_chunk) load_stage(0, 0);
+  for (int c = 0, tg = 0; c < last_chunk;) {
     __syncthreads();  // the previous stage's operand reads are done
-    store_stage(st);
+    store_stage(tg);
     __syncthreads();
-    if (st + 1 < stages) load_stage(st + 1);
-    const int tap0 = st % tap_groups * gt, count = min(gt, nt - tap0);
+    const int count = min(gt, nt - tg * gt);
+    if (++tg == tap_groups) tg = 0, ++c;
+    if (c < last_chunk) load_stage(c, tg);
     for (int k = 0; k < count; ++k) {
       // tap k's input row for position u: d_step < 0 stages the last tap's rows first
       const int shift = d_step < 0 ? (count - 1 - k) * -d_step : k * d_step;
@@ -379,31 +382,86 @@ int launch_tile(MfmaParams p, int max_taps, int reach_step, hipStream_t stream) 
   return OMNI_OK;
 }
 
-template <typename T, bool VX, bool VW>
-int launch_tiles(const MfmaParams& p, int max_taps, int reach_step, hipStream_t stream) {
-  // The tile of the least time: rounds of 256 workgroups times a stage's cost, its padded columns
-  // and positions included, in units of 16 x 16 accumulators plus the staging a tile of any size
-  // pays (kFixed, fitted to the measurements above: float32's MFMAs take 8 times as long).
-  constexpr int kFixed = sizeof(T) == 4 ? 4 : 16;
-  constexpr int tiles[][2] = {{96, 128}, {64, 128}, {32, 128}, {96, 64}, {64, 64}, {32, 32}};
+// The choice between this kernel and one thread per output (conv_general.hip) compares estimates of
+// both at this many rows, whatever the call's own number: the two sum in different orders, and a
+// row's result must not depend on the rows beside it.
+constexpr int kEstimateRows = 16;
+
+// One thread per output, us: its chain of dependent loads, and the loads' traffic at the 64-byte
+// lines that a wave's 64 weights and inputs spread over.
+inline double estimate_scalar(const MfmaParams& p, int max_taps, int size) {
+  const GeneralParams& g = p.g;
+  const double outputs = 1e-6 * kEstimateRows * g.length_out * g.c_out;
+  const double macs = (double)g.taps / p.phases * p.cin_g;  // of an output
+  const double wave_groups = fmin((double)g.groups, fmax(1, 64.0 / p.cout_g));
+  const double wave_pos = fmax(1, 64.0 / g.c_out);
+  const double weights = p.transposed
+      ? wave_groups * fmax(1, (double)p.cout_g * g.taps * size / 64)
+      : 64 / wave_pos * fmin(1, (double)p.cin_g * g.taps * size / 64);
+  const double lines = fmin(64, weights + wave_groups * wave_pos * fmin(1, p.cin_g * size / 64.0));
+  const double chain = 0.1 * max_taps * p.cin_g + (p.transposed ? 0.29 * g.taps : 0);
+  return 2.1 + chain + outputs * (2.9 + 0.68 * g.taps + macs * (0.33 + 1.45 * lines / 64) *
+                                                            (size == 4 ? 1.16 : 1));
+}
+
+constexpr int kTiles[6][2] = {{96, 128}, {64, 128}, {32, 128}, {96, 64}, {64, 64}, {32, 32}};
+
+// Workgroups of tile k at `rows` rows.
+inline int64_t tile_workgroups(const MfmaParams& p, int k, int64_t rows) {
+  return (int64_t)((p.u_count + kTiles[k][1] - 1) / kTiles[k][1]) *
+         ((p.cout_g + kTiles[k][0] - 1) / kTiles[k][0]) * p.phases * p.g.groups * rows;
+}
+
+// The tile of the least time: rounds of 256 workgroups times a stage's cost, its padded columns
+// and positions included, in units of 16 x 16 accumulators plus the staging a tile of any size
+// pays (fitted to the measurements above: float32's MFMAs take 8 times as long). -1: none fits.
+inline int pick_tile(const MfmaParams& p, int64_t rows, int size) {
   int best = -1;
   int64_t least = 0;
   for (int k = 0; k < 6; ++k) {
-    const int bco = tiles[k][0], bp = tiles[k][1];
-    if ((int64_t)(bp - 1) * p.u_step + 1 > kMaxRows) continue;
-    const int64_t wgs = (int64_t)((p.u_count + bp - 1) / bp) * ((p.cout_g + bco - 1) / bco) *
-                        p.phases * p.g.groups * p.g.batch;
-    const int64_t cost = ((wgs + 255) / 256) * (bco * bp / 256 + kFixed);
+    if ((int64_t)(kTiles[k][1] - 1) * p.u_step + 1 > kMaxRows) continue;
+    const int64_t cost = ((tile_workgroups(p, k, rows) + 255) / 256) *
+                         (kTiles[k][0] * kTiles[k][1] / 256 + (size == 4 ? 4 : 16));
     if (best < 0 || cost < least) best = k, least = cost;
   }
-  switch (best) {
+  return best;
+}
+
+// This kernel on the tile k, us: a workgroup's setup, its stages and their MFMAs, one workgroup after
+// another on each CU.
+inline double estimate_tile(const MfmaParams& p, int k, int max_taps, int reach_step,
+                            int stage_taps, int size) {
+  const int base = (kTiles[k][1] - 1) * p.u_step + 1;
+  int taps = max_taps < stage_taps ? max_taps : stage_taps;
+  if (reach_step && (kMaxRows - base) / reach_step + 1 < taps) taps = (kMaxRows - base) / reach_step + 1;
+  const double chunks = (p.cin_g * size + kRowBytes - 1) / kRowBytes;
+  const double stages = chunks * ((max_taps + taps - 1) / taps);
+  const double workgroup = 0.45 + stages * (size == 4 ? 0.39 : 0.61) +
+                           chunks * max_taps * (kTiles[k][0] * kTiles[k][1] / 256) *
+                               (size == 4 ? 0.039 : 0.025);
+  return 3.1 + workgroup * fmax(1, tile_workgroups(p, k, kEstimateRows) / (256 * 1.3));
+}
+
+template <typename T, bool VX, bool VW>
+int launch_tiles(const MfmaParams& p, int max_taps, int reach_step, hipStream_t stream) {
+  constexpr int size = sizeof(T);
+  const int fit = pick_tile(p, kEstimateRows, size);
+  if (fit < 0) return OMNI_ERR_UNSUPPORTED;
+  // Many small workgroups of little work each (grouped convs of a few positions, transposed convs
+  // with fewer taps than phases) take longer than one thread per output: 58 rows of 2 positions,
+  // 64 groups of 24 -> 5 channels, 2 taps at stride 8 are 29 696 workgroups, 88 us against 6.9.
+  // Over 1 636 drawn forms at a few hundred products and fewer an output the choice lies within
+  // 1.6 % of the better kernel in the mean (this kernel always: 4.4 %).
+  constexpr int stage_taps = GeneralTile<T, 2, 2, 1, 1, VX, VW>::G;
+  if (estimate_scalar(p, max_taps, size) < estimate_tile(p, fit, max_taps, reach_step, stage_taps, size))
+    return OMNI_ERR_UNSUPPORTED;
+  switch (pick_tile(p, p.g.batch, size)) {
     case 0: return launch_tile<T, 2, 2, 3, 4, VX, VW>(p, max_taps, reach_step, stream);
     case 1: return launch_tile<T, 2, 2, 2, 4, VX, VW>(p, max_taps, reach_step, stream);
     case 2: return launch_tile<T, 1, 4, 2, 2, VX, VW>(p, max_taps, reach_step, stream);
     case 3: return launch_tile<T, 2, 2, 3, 2, VX, VW>(p, max_taps, reach_step, stream);
     case 4: return launch_tile<T, 2, 2, 2, 2, VX, VW>(p, max_taps, reach_step, stream);
-    case 5: return launch_tile<T, 2, 2, 1, 1, VX, VW>(p, max_taps, reach_step, stream);
-    default: return OMNI_ERR_UNSUPPORTED;
+    default: return launch_tile<T, 2, 2, 1, 1, VX, VW>(p, max_taps, reach_step, stream);
   }
 }
 
@@ -420,7 +478,7 @@ int launch_mfma(const GeneralParams& g, bool transposed, hipStream_t stream) {
   if (g.length_in < 1 || g.length_in > kBig || g.length_out > kBig || g.c_in > kBig || g.c_out > kBig ||
       g.taps > kBig || g.stride > kBig || g.dilation > kBig || g.pad_left > kBig ||
       g.taps * g.dilation > kBig || (g.length_out + g.pad_left) > kBig ||
-      (g.length_out + 128) * g.stride > kBig)
+      (g.length_out + 128) * g.stride > kBig || (transposed && g.stride > 32768))
     return OMNI_ERR_UNSUPPORTED;
   constexpr int64_t kLimit = 0x7fffffffLL;  // byte offsets are 32-bit
   if (g.x_st > kLimit || g.x_sc > kLimit || g.w_s0 > kLimit || g.w_s1 > kLimit || g.w_s2 > kLimit)
@@ -443,6 +501,14 @@ int launch_mfma(const GeneralParams& g, bool transposed, hipStream_t stream) {
     int a = (int)g.stride, c = (int)(g.dilation % g.stride);
     while (c) { const int m = a % c; a = c; c = m; }
     const int j_step = (int)g.stride / a;
+    p.s_dil_gcd = a;
+    // 1 / (dilation / a) mod j_step (Euclid)
+    int64_t r0 = j_step, r1 = g.dilation / a % j_step, t0 = 0, t1 = 1;
+    while (r1) {
+      const int64_t q = r0 / r1, r = r0 - q * r1, t = t0 - q * t1;
+      r0 = r1, r1 = r, t0 = t1, t1 = t;
+    }
+    p.dil_inv = (int)(t0 < 0 ? t0 + j_step : t0);
     max_taps = ((int)g.taps + j_step - 1) / j_step;
     reach_step = (int)g.dilation / a;
     p.phases = (int)g.stride;

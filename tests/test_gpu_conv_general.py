@@ -161,3 +161,62 @@ def test_a_tap_outside_the_row_adds_nothing_whatever_its_weight(gpu, dtype, bad,
         got[:, :, channel] = want[:, :, channel]
         assert torch.equal(got, want)
     assert missed > 0  # outputs that a tap does not reach
+
+
+# forms on both sides of the line between the matrix cores and one thread per output
+LINE = [
+    (58, 2, 1536, 320, 2, 64, 8, 1, 0, True),   # 64 groups, 8 phases, 2 taps: tiny workgroups
+    (62, 3, 128, 1536, 1, 32, 8, 3, 0, True),
+    (46, 9, 512, 128, 2, 32, 8, 1, 3, True),
+    (21, 51, 192, 128, 1, 32, 4, 1, 0, False),
+    (3, 171, 768, 256, 1, 64, 1, 1, 0, False),
+    (40, 8, 64, 64, 3, 16, 1, 1, 2, False),
+    (9, 300, 48, 48, 4, 2, 2, 1, 1, True),
+    (12, 40, 96, 96, 7, 1, 1, 3, 6, False),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("batch,length,c_in,c_out,taps,groups,stride,dilation,pad,transposed", LINE)
+def test_a_row_does_not_depend_on_the_rows_beside_it(gpu, dtype, batch, length, c_in, c_out, taps,
+                                                     groups, stride, dilation, pad, transposed):
+    """The kernel is chosen without regard to the batch, so a row has the same bits alone."""
+    x, w, b = draw(gpu, dtype, batch, length, c_in, c_out, taps, groups, transposed)
+    reach = dilation * (taps - 1)
+    out = (length - 1) * stride + reach + 1 - pad if transposed else (length + pad - reach - 1) // stride + 1
+    kw = dict(groups=groups, stride=stride, dilation=dilation, transposed=transposed)
+    got = _general(x, w, b, c_out=c_out, pad_left=pad, length_out=out, **kw)
+    check(got, x, w, b, pad=pad, **kw)
+    for rows in (slice(0, 1), slice(batch - 1, batch), slice(1, 3)):
+        assert torch.equal(_general(x[rows], w, b, c_out=c_out, pad_left=pad, length_out=out, **kw),
+                           got[rows])
+
+
+@pytest.mark.parametrize("batch,length,c_in,c_out,taps,groups,stride,dilation,pad,transposed", LINE[:3])
+def test_many_small_groups_are_not_a_workgroup_each(gpu, batch, length, c_in, c_out, taps, groups,
+                                                    stride, dilation, pad, transposed):
+    """As matrix-core tiles of a few outputs each these took 7 to 20 times a single row's time (23 and
+    more us); one thread per output takes 1.5 to 3 times (7 to 12 us)."""
+    def microseconds(rows):
+        x, w, b = draw(gpu, torch.float32, rows, length, c_in, c_out, taps, groups, transposed)
+        out = (length - 1) * stride + dilation * (taps - 1) + 1 - pad
+        run = lambda: _general(x, w, b, c_out=c_out, pad_left=pad, length_out=out, groups=groups,
+                               stride=stride, dilation=dilation, transposed=transposed)
+        side = torch.cuda.Stream()
+        with torch.cuda.stream(side):
+            run()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            kept = [run() for _ in range(20)]
+        start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        best = float("inf")
+        for _ in range(10):
+            start.record()
+            graph.replay()
+            end.record()
+            torch.cuda.synchronize()
+            best = min(best, start.elapsed_time(end) * 1e3 / len(kept))
+        return best
+
+    assert microseconds(batch) <= 4.5 * microseconds(1)
