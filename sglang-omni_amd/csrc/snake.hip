@@ -87,7 +87,9 @@ __device__ __forceinline__ void st8(void* p, int64_t i, const float (&v)[8]) {
 // expression: one element per thread spent more instructions on its two 64-bit divisions than on
 // the activation. Bound by sinf. Channels and strides multiples of 8, pointers 16-byte aligned,
 // fewer than 2^31 groups of eight. 3.69 M float16 elements: 14.3 -> 9.1 us, with the residual and
-// the sum 16.4 -> 11.7.
+// the sum 16.4 -> 11.7. A thread's eight sinf one after another are its time where there are too few
+// elements to fill the GPU, so calls below kEightFrom keep one element per thread: a few thousand
+// elements 2.4 us one-wide, 3.2 eight-wide; 345 600 3.4 and 3.7; 801 312 4.6 and 4.1.
 template <int DT, int PDT>
 __global__ void __launch_bounds__(256) bias_snake_beta8_kernel(
     const void* conv, int64_t conv_sb, uint32_t groups, uint32_t row_groups,
@@ -173,6 +175,8 @@ __global__ void __launch_bounds__(256) snake_beta_params_kernel(
 
 bool half_like(int dt) { return dt == OMNI_DTYPE_BF16 || dt == OMNI_DTYPE_F16; }
 
+constexpr int64_t kEightFrom = 256 * 2048;  // eight-wide gives each of 256 CUs a workgroup
+
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 template <int DT, int PDT>
@@ -182,7 +186,7 @@ int launch_bsb_as(const void* conv, int64_t conv_sb, int64_t batch, int64_t leng
                   int64_t out_sb, hipStream_t s) {
   const int64_t n = batch * length * channels;
   // (a row stride matters from the second row on)
-  const bool eight = channels % 8 == 0 && (batch == 1 || (conv_sb % 8 == 0 && out_sb % 8 == 0)) &&
+  const bool eight = n >= kEightFrom && channels % 8 == 0 && (batch == 1 || (conv_sb % 8 == 0 && out_sb % 8 == 0)) &&
                      n / 8 < 0x7fffff00LL && aligned16(conv) && aligned16(bias) &&
                      aligned16(alpha_scale) && aligned16(inverse_beta) && aligned16(residual) &&
                      aligned16(sum_out) && aligned16(out);
