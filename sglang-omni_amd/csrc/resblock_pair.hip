@@ -352,13 +352,14 @@ int launch_as(const ConvParams& p1, const ConvParams& p2, hipStream_t stream) {
 }
 
 // GP: the 16-row groups a wave takes through a conv at once (as many as the registers hold: with
-// the float16 stream four at k = 11, two otherwise).
+// the float16 stream four at k = 11, two otherwise, but one at k = 3 with the float32 mix, where two
+// spill 20 registers at two workgroups a CU: 4 x 325 366 positions 167 us, with one 130).
 template <int K, int OCC, int GP16>
 int launch(const ConvParams& p1, const ConvParams& p2, hipStream_t s) {
   if (p2.r_f16)
     return p2.mix_a ? launch_as<K, OCC, GP16, true, true>(p1, p2, s)
                     : launch_as<K, OCC, GP16, true, false>(p1, p2, s);
-  return p2.mix_a ? launch_as<K, OCC, 2, false, true>(p1, p2, s)
+  return p2.mix_a ? launch_as<K, OCC, K == 3 ? 1 : 2, false, true>(p1, p2, s)
                   : launch_as<K, OCC, 2, false, false>(p1, p2, s);
 }
 
