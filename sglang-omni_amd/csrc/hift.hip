@@ -281,7 +281,8 @@ __device__ __forceinline__ void tail_sincos(float p, float& sn, float& cs) {
 // frames' 72 components from LDS (16 us of LDS traffic at the size below) and multiplied them on
 // the VALU. An output's sum order is fixed: components in the MFMA's order within a frame, then
 // overlaps. Bound by: the tail's VALU work per (frame, bin); the inverse, HBM.
-// Measured, 16 x 240 000 samples: tail 43.8 -> 28.7 us (84 MB: 2.9 TB/s), inverse 47 -> 23.4 us
+// Measured, 16 x 240 000 samples: tail 43.8 -> 28.7 us (84 MB: 2.9 TB/s), inverse 47 -> 23.4
+// us; 3 x 5 frames 3.5 and 4.0 -> 3.8 (5.6 and 4.4 with the tail's functions over the whole window).
 constexpr int kInv16Quads = kThreads;                  // quads of samples per workgroup
 constexpr int kInv16Samples = 4 * kInv16Quads;
 constexpr int kInv16Frames = kInv16Quads + 3;          // frames that reach them
@@ -325,16 +326,17 @@ __global__ void __launch_bounds__(kThreads) overlap_add_inverse16_kernel(const I
       }
     }
     __syncthreads();
-    int j = tid / BINS, b = tid - j * BINS;
+    // (the row's own frames only: what lies in LDS for the others meets its own column of the
+    // product, which nothing reads)
+    int j = lo + tid / BINS, b = tid % BINS;
 #pragma unroll 3
-    for (int e = tid; e < kInv16Frames * BINS; e += kThreads) {
+    for (int e = lo * BINS + tid; e < hi * BINS; e += kThreads) {
       float* s = spec + j * COMPS + b;
       const float mag = fminf(tail_exp(s[0]), p.mag_clip);
       float sn, cs;
       tail_sincos(tail_sin(s[BINS]), sn, cs);
-      const bool real = j >= lo && j < hi;
-      s[0] = real ? mag * cs : 0.f;
-      s[BINS] = real ? mag * sn : 0.f;
+      s[0] = mag * cs;
+      s[BINS] = mag * sn;
       j += kThreads / BINS;
       b += kThreads % BINS;
       if (b >= BINS) b -= BINS, ++j;
@@ -366,7 +368,7 @@ __global__ void __launch_bounds__(kThreads) overlap_add_inverse16_kernel(const I
   for (int k = 0; k < GROUPS; ++k) {
     acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int g = wave + k * (kThreads / 64);
-    if (g >= kInv16Groups) break;
+    if (g * 16 >= hi) break;
     const float* sp = spec + (g * 16 + ln) * COMPS + lq;
 #pragma unroll
     for (int s = 0; s < 5; ++s) {
@@ -378,7 +380,7 @@ __global__ void __launch_bounds__(kThreads) overlap_add_inverse16_kernel(const I
 #pragma unroll
   for (int k = 0; k < GROUPS; ++k) {
     const int g = wave + k * (kThreads / 64);
-    if (g < kInv16Groups) parts[lq * ROWS + g * 16 + ln] = acc[k];
+    if (g * 16 < hi) parts[lq * ROWS + g * 16 + ln] = acc[k];
   }
   __syncthreads();
   const int64_t i = i0 + 4 * tid;
