@@ -402,6 +402,30 @@ int omni_residual_stack_coefficients(const omni_residual_stack_args* a, float* t
 int omni_residual_stack(const omni_residual_stack_args* args, omni_stream_t stream);
 
 /*
+ * How a launch stages its rows, chosen by the sizes; every form gives the same bits.
+ *   OMNI_STACK_FORM_SWEEP    a workgroup runs consecutive tiles of 384 staged rows of one row (rows
+ *                            longer than a tile, at most 3 units)
+ *   OMNI_STACK_FORM_ROWS384  tiles of 384 staged rows, each with its own halo: parts of a long row, or
+ *                            several short rows
+ *   OMNI_STACK_FORM_ROWS256, OMNI_STACK_FORM_ROWS128  the same with 256 and 128 staged rows
+ * omni_residual_stack_with runs the named form (OMNI_ERR_UNSUPPORTED where it cannot hold the call);
+ * omni_residual_stack_plan reports, without launching, the form that omni_residual_stack (form =
+ * OMNI_STACK_FORM_AUTO) or omni_residual_stack_with would run and its workgroups (0 for an empty
+ * call).
+ */
+enum {
+  OMNI_STACK_FORM_AUTO = 0,
+  OMNI_STACK_FORM_SWEEP = 1,
+  OMNI_STACK_FORM_ROWS384 = 2,
+  OMNI_STACK_FORM_ROWS256 = 3,
+  OMNI_STACK_FORM_ROWS128 = 4
+};
+
+int omni_residual_stack_with(const omni_residual_stack_args* args, int form, omni_stream_t stream);
+int omni_residual_stack_plan(const omni_residual_stack_args* args, int form, int* form_out,
+                             int64_t* workgroups);
+
+/*
  * Conv from channels-last activations to one output channel, stride 1, undilated:
  *   u = in_act(x) (OMNI_ACTIVATION_NONE or _SNAKE with per-channel in_act_a / in_act_b)
  *   out[b, i] = act(bias + sum_{j < taps} sum_c weight[j * channels + c] * u[b, i + j - left_pad, c])

@@ -25,7 +25,7 @@
 //     read.
 //   * long rows (sweep): a workgroup runs consecutive tiles of one stream row, and each operand's
 //     last halo rows pass from one tile to the next through LDS instead of being recomputed; where
-//     the sweep would leave most CUs idle, tiles of 256 or 128 staged rows recompute their halo.
+//     the sweep would leave CUs idle, tiles of 384, 256 or 128 staged rows recompute their halo.
 //   * streaming: rows left of position 0 of a stream row take each unit's own history copy (or
 //     zeros), and the workgroup that owns the last 6 * d positions of a row writes them as the
 //     unit's new history, as the one-unit kernel does.
@@ -887,17 +887,14 @@ using Stack96Dma = StackTile<96, 1, 8, 3>;
 using Stack96Sweep = StackTile<96, 1, 8, 3, true>;
 using Stack96Dma8 = StackTile<96, 1, 8, 3, false, true>;
 using Stack96Sweep8 = StackTile<96, 1, 8, 3, true, true>;
-// The tiled form at 256 and 128 staged rows (2 and 1 position tiles a wave), for calls that give
-// the sweep few workgroups.
+// The tiled form at 256 and 128 staged rows (2 and 1 position tiles a wave), for calls of few
+// positions.
 template <int TP, bool W8>
 using Stack96Tiled = StackTile<96, 1, 8, TP, false, W8>;
 static_assert(Stack96Sweep::lds_bytes() <= 160 * 1024, "the sweep form fits the CU's LDS");
 static_assert(Stack96Sweep8::lds_bytes() <= Stack96Sweep::lds_bytes() &&
               Stack96Dma8::R == Stack96Dma::R && Stack96Sweep8::R == Stack96Dma::R,
               "E4M3 weights take the bf16 forms' tiles");
-
-// How a launch stages its rows: the sweep, or tiles of 384, 256 or 128 staged rows.
-enum StackForm { kFormSweep, kForm384, kForm256, kForm128 };
 
 template <int TP, bool W_FP8, bool SWEEP>
 int launch_stack_form(const StackParams& p, int grid, hipStream_t stream) {
@@ -911,15 +908,15 @@ int launch_stack_form(const StackParams& p, int grid, hipStream_t stream) {
 }
 
 template <bool W_FP8>
-int launch_stack96(const StackParams& p, int grid, StackForm form, hipStream_t stream) {
+int launch_stack96(const StackParams& p, int grid, int form, hipStream_t stream) {
   switch (form) {
-    case kFormSweep: return launch_stack_form<3, W_FP8, true>(p, grid, stream);
-    case kForm384: return launch_stack_form<3, W_FP8, false>(p, grid, stream);
-    case kForm256: return launch_stack_form<2, W_FP8, false>(p, grid, stream);
+    case OMNI_STACK_FORM_SWEEP: return launch_stack_form<3, W_FP8, true>(p, grid, stream);
+    case OMNI_STACK_FORM_ROWS384: return launch_stack_form<3, W_FP8, false>(p, grid, stream);
+    case OMNI_STACK_FORM_ROWS256: return launch_stack_form<2, W_FP8, false>(p, grid, stream);
     default: return launch_stack_form<1, W_FP8, false>(p, grid, stream);
   }
 }
-extern template int launch_stack96<false>(const StackParams&, int, StackForm, hipStream_t);
-extern template int launch_stack96<true>(const StackParams&, int, StackForm, hipStream_t);
+extern template int launch_stack96<false>(const StackParams&, int, int, hipStream_t);
+extern template int launch_stack96<true>(const StackParams&, int, int, hipStream_t);
 
 }  // namespace omni_stack

@@ -40,6 +40,16 @@ void coef_sources(const omni_residual_stack_args* a, bool fp8, omni_stack::Stack
   p.out_b = a->out_act_b;
 }
 
+// Staged rows per tile of a form (both weight formats).
+int64_t form_rows(int form) {
+  using namespace omni_stack;
+  switch (form) {
+    case OMNI_STACK_FORM_ROWS256: return Stack96Tiled<2, false>::R;
+    case OMNI_STACK_FORM_ROWS128: return Stack96Tiled<1, false>::R;
+    default: return Stack96Dma::R;
+  }
+}
+
 }  // namespace
 
 extern "C" int omni_residual_stack_coefficients(const omni_residual_stack_args* a, float* table,
@@ -66,8 +76,14 @@ extern "C" int omni_residual_stack_coefficients(const omni_residual_stack_args* 
   return OMNI_OK;
 }
 
-extern "C" int omni_residual_stack(const omni_residual_stack_args* a, omni_stream_t stream) {
+namespace {
+
+// form_want: OMNI_STACK_FORM_AUTO or the form to run; form_out / workgroups_out report the choice.
+int stack_entry(const omni_residual_stack_args* a, int form_want, bool launch, int* form_out,
+                int64_t* workgroups_out, omni_stream_t stream) {
   using namespace omni_stack;
+  if (form_want < OMNI_STACK_FORM_AUTO || form_want > OMNI_STACK_FORM_ROWS128)
+    return OMNI_ERR_INVALID_ARG;
   if (!a || !a->x || !a->out_act_a || !a->out_act_b) return OMNI_ERR_INVALID_ARG;
   const bool fin = a->final_weight != nullptr;
   if (!a->out && !fin) return OMNI_ERR_INVALID_ARG;
@@ -130,7 +146,11 @@ extern "C" int omni_residual_stack(const omni_residual_stack_args* a, omni_strea
   }
   if (any_hist && (!a->slot_index || !a->slot_parity || a->hist_num_slots < 1))
     return OMNI_ERR_INVALID_ARG;
-  if (a->batch == 0 || a->length == 0) return OMNI_OK;
+  if (a->batch == 0 || a->length == 0) {
+    if (form_out) *form_out = OMNI_STACK_FORM_AUTO;
+    if (workgroups_out) *workgroups_out = 0;
+    return OMNI_OK;
+  }
   const int64_t R = Stack96Dma::R;  // staged rows per tile (both weight formats)
   if (H + 16 > R) return OMNI_ERR_UNSUPPORTED;
 
@@ -211,24 +231,54 @@ extern "C" int omni_residual_stack(const omni_residual_stack_args* a, omni_strea
     p.fin_o_sb = a->final_out_stride_b;
   }
 
-  // Long rows: the sweep (each workgroup runs consecutive tiles of one row,
-  // the causal halo staged once per workgroup instead of once per tile), one workgroup per
-  // compute unit where the rows allow. Otherwise long rows take tiles inside one row, as many as
-  // the staged rows need, evened out; short rows as many whole rows (each with its halo) as the
-  // staged rows hold.
-  int64_t grid;
-  StackForm form = kForm384;
-  bool sweep = false;
-  if (L + H > R && a->num_units <= kSweepUnits) {
-    int64_t halo_rows = fin ? a->final_taps - 1 : 0;
-    bool fits = halo_rows <= kSweepGuard;
-    for (int k = 0; k < a->num_units; ++k) {
-      halo_rows += 6 * a->units[k].dilation;
-      fits = fits && 6 * a->units[k].dilation <= kSweepGuard;
-    }
-    sweep = fits && halo_rows <= kSweepHaloRows;
+  // Short rows: as many whole rows (each with its halo) per tile as the staged rows hold. Long rows:
+  // the sweep (each workgroup runs consecutive tiles of one row, the causal halo staged once per
+  // workgroup instead of once per tile), one workgroup per compute unit where the rows allow, or
+  // tiles inside one row, as many as the staged rows need, evened out.
+  const int64_t cus = compute_units();
+  int64_t halo_rows = fin ? a->final_taps - 1 : 0;
+  bool sweeps = L + H > R && a->num_units <= kSweepUnits && halo_rows <= kSweepGuard;
+  for (int k = 0; k < a->num_units; ++k) {
+    halo_rows += 6 * a->units[k].dilation;
+    sweeps = sweeps && 6 * a->units[k].dilation <= kSweepGuard;
   }
-  if (sweep) {
+  sweeps = sweeps && halo_rows <= kSweepHaloRows;
+  int64_t segments = B >= cus ? 1 : cus / B;
+  // at least two tiles per segment, or the sweep saves no halo
+  const int64_t max_segments = (L + 2 * R - 1) / (2 * R);
+  segments = segments < 1 ? 1 : (segments > max_segments ? max_segments : segments);
+  const int64_t sweep_positions = (L + segments - 1) / segments;
+
+  int form = form_want;
+  if (form == OMNI_STACK_FORM_AUTO) {
+    form = OMNI_STACK_FORM_ROWS384;
+    if (sweeps) {
+      // The least of four estimates, us. The sweep: rounds of its workgroups, each full tile of 384
+      // rows (the halo among them) and the last, shorter one after another; it saves the halos, but
+      // gives few positions few workgroups. Tiles: rounds of them, each staging the whole halo.
+      // Measured, us, sweep / 384 / 256 / 128 rows: 1 x 7 680 positions 129 / 55 / 40 / 29, 16 x
+      // 7 680 131 / 106 / 117 / 275, 48 x 2 371 100 / 106 / 118 / 274, 223 x 400 86 / 102 / 116 / 230,
+      // 174 x 2 000 282 / 265 / 340 / 653, 1 x 480 000 292 / 365 / 405 / 909. Over 324 sizes the choice
+      // takes 0.03 % more than the best form in the mean, 4 % at most.
+      const int64_t sweep_rows = sweep_positions + H;
+      double least = (double)((B * segments + cus - 1) / cus) *
+                     (14 + 51.0 * (sweep_rows / R) + (sweep_rows % R ? 28 : 0));
+      form = OMNI_STACK_FORM_SWEEP;
+      const struct { int form; double fixed, round; } tiled[] = {{OMNI_STACK_FORM_ROWS384, 2, 52},
+                                                                 {OMNI_STACK_FORM_ROWS256, 4, 37.5},
+                                                                 {OMNI_STACK_FORM_ROWS128, 5, 24.5}};
+      for (const auto& f : tiled) {
+        const int64_t rows = form_rows(f.form);
+        if (H + 32 > rows) continue;
+        const int64_t per_row = (L + (rows - H) - 1) / (rows - H);
+        const double us = f.fixed + f.round * ((B * per_row + cus - 1) / cus);
+        if (us < least) least = us, form = f.form;
+      }
+    }
+  }
+  int64_t grid;
+  if (form == OMNI_STACK_FORM_SWEEP) {
+    if (!sweeps) return OMNI_ERR_UNSUPPORTED;
     int off = 0;
     for (int k = 0; k <= a->num_units; ++k) {
       const int rows_k = k < a->num_units ? (int)(6 * a->units[k].dilation)
@@ -237,49 +287,45 @@ extern "C" int omni_residual_stack(const omni_residual_stack_args* a, omni_strea
       p.halo_off[k] = off;
       off += rows_k;
     }
-    const int64_t cus = compute_units();
-    int64_t segments = B >= cus ? 1 : cus / B;
-    // at least two tiles per segment, or the sweep saves no halo
-    const int64_t max_segments = (L + 2 * R - 1) / (2 * R);
-    segments = segments < 1 ? 1 : (segments > max_segments ? max_segments : segments);
     p.sweep_segments = (int)segments;
-    p.sweep_positions = (int)((L + segments - 1) / segments);
+    p.sweep_positions = (int)sweep_positions;
     grid = B * segments;
-    form = kFormSweep;
-    // Few positions give the sweep few workgroups, each running two and more tiles one after the
-    // other (56 to 65 us each): smaller tiles, each with the whole stack's halo, spread them over the
-    // GPU. Measured, us, sweep / 256 rows / 128 rows: 1 x 7 680 positions 129 / 40 / 29, 1 x
-    // 23 040 130 / 41 / 80, 8 x 7 680 131 / 79 / 152, 16 x 7 680 131 / 117 / 275, 1 x 480 000 279
-    // / 412 / 1 060.
-    const int64_t tiles = (p.sweep_positions + R - 1) / R;
-    double least = 64.0 * tiles;
-    const struct { StackForm form; int64_t rows; double us; } small[] = {
-        {kForm256, Stack96Tiled<2, false>::R, 40.0}, {kForm128, Stack96Tiled<1, false>::R, 28.0}};
-    for (const auto& f : small) {
-      if (H + 32 > f.rows) continue;
-      const int64_t per_row = (L + (f.rows - H) - 1) / (f.rows - H);
-      const double us = f.us * ((B * per_row + cus - 1) / cus);
-      if (us < least) {
-        least = us;
-        form = f.form;
-        p.seg_len = (int)((L + per_row - 1) / per_row);
-        p.tiles_per_row = (int)((L + p.seg_len - 1) / p.seg_len);
-        grid = B * p.tiles_per_row;
-      }
-    }
-  } else if (L + H > R) {
-    const int64_t tiles = (L + (R - H) - 1) / (R - H);
-    p.seg_len = (int)((L + tiles - 1) / tiles);
-    p.tiles_per_row = (int)((L + p.seg_len - 1) / p.seg_len);
-    grid = B * p.tiles_per_row;
   } else {
-    p.seg_len = (int)L;
-    p.tiles_per_row = 0;
-    p.rows_per_tile = (int)(R / (L + H));
-    grid = (B + p.rows_per_tile - 1) / p.rows_per_tile;
+    const int64_t rows = form_rows(form);
+    if (H + 16 > rows) return OMNI_ERR_UNSUPPORTED;
+    if (L + H > rows) {
+      const int64_t tiles = (L + (rows - H) - 1) / (rows - H);
+      p.seg_len = (int)((L + tiles - 1) / tiles);
+      p.tiles_per_row = (int)((L + p.seg_len - 1) / p.seg_len);
+      grid = B * p.tiles_per_row;
+    } else {
+      p.seg_len = (int)L;
+      p.tiles_per_row = 0;
+      p.rows_per_tile = (int)(rows / (L + H));
+      grid = (B + p.rows_per_tile - 1) / p.rows_per_tile;
+    }
   }
   if (grid > 0x7fffffffLL) return OMNI_ERR_UNSUPPORTED;
+  if (form_out) *form_out = form;
+  if (workgroups_out) *workgroups_out = grid;
+  if (!launch) return OMNI_OK;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   return fp8 ? launch_stack96<true>(p, (int)grid, form, s)
              : launch_stack96<false>(p, (int)grid, form, s);
+}
+
+}  // namespace
+
+extern "C" int omni_residual_stack(const omni_residual_stack_args* a, omni_stream_t stream) {
+  return stack_entry(a, OMNI_STACK_FORM_AUTO, true, nullptr, nullptr, stream);
+}
+
+extern "C" int omni_residual_stack_with(const omni_residual_stack_args* a, int form,
+                                        omni_stream_t stream) {
+  return stack_entry(a, form, true, nullptr, nullptr, stream);
+}
+
+extern "C" int omni_residual_stack_plan(const omni_residual_stack_args* a, int form, int* form_out,
+                                        int64_t* workgroups) {
+  return stack_entry(a, form, false, form_out, workgroups, nullptr);
 }

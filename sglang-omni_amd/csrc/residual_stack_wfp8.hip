@@ -3,6 +3,6 @@
 
 namespace omni_stack {
 
-template int launch_stack96<true>(const StackParams&, int, StackForm, hipStream_t);
+template int launch_stack96<true>(const StackParams&, int, int, hipStream_t);
 
 }  // namespace omni_stack

@@ -50,6 +50,10 @@ CONV_KERNEL_NAMES = {CONV_KERNEL_DMA: "dma", CONV_KERNEL_STAGED: "staged",
                      CONV_KERNEL_STAGED11: "staged11", CONV_KERNEL_FUSED_UNIT: "fused_unit",
                      CONV_KERNEL_SMALL: "small", CONV_KERNEL_DMA_MID: "dma_mid"}
 
+# how omni_residual_stack stages its rows (omni_residual_stack_plan / omni_residual_stack_with)
+(STACK_FORM_AUTO, STACK_FORM_SWEEP, STACK_FORM_ROWS384, STACK_FORM_ROWS256,
+ STACK_FORM_ROWS128) = range(5)
+
 
 class ConvArgs(ctypes.Structure):
     """Mirror of ``omni_conv_args`` in include/omni_codec.h (field order and types match)."""
@@ -212,6 +216,9 @@ SIGNATURES: dict[str, list] = {
     "omni_conv1d_plan": [ctypes.POINTER(ConvArgs), _INT, _INT, ctypes.POINTER(_INT),
                          ctypes.POINTER(_INT), ctypes.POINTER(_INT), ctypes.POINTER(_I64)],
     "omni_residual_stack": [ctypes.POINTER(ResidualStackArgs), _PTR],
+    "omni_residual_stack_with": [ctypes.POINTER(ResidualStackArgs), _INT, _PTR],
+    "omni_residual_stack_plan": [ctypes.POINTER(ResidualStackArgs), _INT, ctypes.POINTER(_INT),
+                                 ctypes.POINTER(_I64)],
     "omni_residual_stack_coefficients": [ctypes.POINTER(ResidualStackArgs), _PTR, _I64, _PTR],
     "omni_single_output_conv": [_PTR, _INT, _I64, _I64, _I64, _I64, _I64, _INT, _INT, _PTR, _PTR,
                                 _PTR, _PTR, _I64, _I64, _PTR, _PTR, _PTR, _I64, _I64, _INT, _INT,

@@ -543,6 +543,7 @@ def residual_stack(
     history_cold: bool = False,
     final: FinalConv | None = None,
     coef_table: torch.Tensor | None = None,
+    form: int = N.STACK_FORM_AUTO,
 ) -> torch.Tensor:
     """Launch ``omni_residual_stack``: every unit in turn over x [B, L, C] (float32, or a
     float16 residual stream, kept in float32 between the units), then out = Snake(out_a,
@@ -550,7 +551,8 @@ def residual_stack(
     histories[k] is unit k's conv1 history pool [slots, 2, 6 * dilation, C] bf16 (streaming).
     With ``final`` the decoder's conv to one channel runs over out inside the same launch and
     writes final.out [B, 1, L] float32 (out may then be None: the operand stays on chip); returns
-    final.out, else out."""
+    final.out, else out. ``form`` names how the rows are staged (N.STACK_FORM_*, chosen by the sizes
+    unless named; the same bits)."""
     N.require_device(x, out, x_out)
     dev = x.device
     if not 1 <= len(units) <= N.MAX_RESIDUAL_UNITS:
@@ -672,9 +674,38 @@ def residual_stack(
             raise ValueError("coef_table must be stack_coefficients(...) of these units")
         args.coef_table = coef_table.data_ptr()
     lib = N.load_library()
-    N.check(lib.omni_residual_stack(ctypes.byref(args), N.stream_handle(x.device)),
+    N.check(lib.omni_residual_stack_with(ctypes.byref(args), form, N.stream_handle(x.device)),
             "omni_residual_stack")
     return final.out if final is not None else out
+
+
+def plan_stack_shapes(*, batch: int, length: int, dilations: tuple[int, ...], final_taps: int = 0,
+                      fp8: bool = False, form: int = N.STACK_FORM_AUTO) -> tuple[int, int]:
+    """The form (N.STACK_FORM_*) and workgroups of a stack call described by its shapes alone
+    (placeholder aligned addresses; nothing runs, so this works without a GPU)."""
+    fake = 1 << 20
+    args = N.ResidualStackArgs()
+    args.x = args.out_act_a = args.out_act_b = args.out = fake
+    args.x_dtype = N.DTYPE_F16
+    args.batch, args.length, args.channels = batch, length, 96
+    args.x_stride_t = args.out_stride_t = 96
+    args.x_stride_b = args.out_stride_b = length * 96
+    args.weight_dtype = N.DTYPE_FP8_E4M3 if fp8 else N.DTYPE_BF16
+    args.num_units = len(dilations)
+    for k, d in enumerate(dilations):
+        a = args.units[k]
+        a.weight1 = a.weight2 = a.in_act_a = a.in_act_b = a.mid_act_a = a.mid_act_b = fake
+        a.weight1_scale = a.weight2_scale = fake if fp8 else None
+        a.dilation = d
+    if final_taps:
+        args.final_weight = args.final_out = fake
+        args.final_taps, args.final_activation = final_taps, N.ACT_TANH
+        args.final_out_stride_b = length
+    chosen, workgroups = ctypes.c_int(), ctypes.c_int64()
+    N.check(N.load_library().omni_residual_stack_plan(ctypes.byref(args), form, ctypes.byref(chosen),
+                                                      ctypes.byref(workgroups)),
+            "omni_residual_stack_plan")
+    return chosen.value, workgroups.value
 
 
 def stack_coefficients(units: list[ResidualUnitWeights], out_a: torch.Tensor,

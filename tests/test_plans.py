@@ -9,7 +9,7 @@ import ctypes
 import pytest
 
 from sglang_omni_amd import _native as N
-from sglang_omni_amd.kernels.conv import plan_shapes
+from sglang_omni_amd.kernels.conv import plan_shapes, plan_stack_shapes
 from tests.test_gpu_tiles import (
     DMA_LIST,
     FUSED_LIST,
@@ -148,3 +148,40 @@ def test_what_no_tile_serves_the_small_kernel_does_not_either():
     loaded = plan_shapes(batch=64, length=3840, c_in=192, n_cols=192, c_out=192, taps=7,
                          dilation=9, fused_unit=True)
     assert loaded.kernel == N.CONV_KERNEL_FUSED_UNIT
+
+
+@pytest.mark.parametrize("batch,length,form", [
+    # the form measured fastest of the four (us: sweep / 384 / 256 / 128 rows)
+    (1, 310, N.STACK_FORM_ROWS128),       # 84 / 52 / 41 / 29
+    (8, 1500, N.STACK_FORM_ROWS256),      # 131 / 55 / 43 / 56
+    (16, 7680, N.STACK_FORM_ROWS384),     # 131 / 106 / 117 / 275
+    (48, 2371, N.STACK_FORM_SWEEP),       # 100 / 106 / 118 / 274
+    (100, 2371, N.STACK_FORM_SWEEP),      # 180 / 209 / 228 / 556
+    (128, 1000, N.STACK_FORM_SWEEP),      # 102 / 106 / 122 / 299
+    (223, 400, N.STACK_FORM_SWEEP),       # 86 / 102 / 116 / 230
+    (174, 2000, N.STACK_FORM_ROWS384),    # 282 / 265 / 340 / 653
+    (512, 1000, N.STACK_FORM_SWEEP),      # 310 / 405 / 471 / 1137
+    (1, 480000, N.STACK_FORM_SWEEP),      # 292 / 365 / 405 / 909
+    (64, 23040, N.STACK_FORM_SWEEP), (8, 60001, N.STACK_FORM_SWEEP),
+    (64, 12, N.STACK_FORM_ROWS384), (1, 300, N.STACK_FORM_ROWS384),  # whole rows
+])
+def test_the_stack_takes_its_fastest_form(batch, length, form):
+    final = 7 if batch % 2 == 0 else 0
+    chosen, workgroups = plan_stack_shapes(batch=batch, length=length, dilations=(1, 3, 9),
+                                           final_taps=final)
+    assert chosen == form
+    # the named form is the same plan
+    assert plan_stack_shapes(batch=batch, length=length, dilations=(1, 3, 9), final_taps=final,
+                             form=form) == (chosen, workgroups)
+
+
+def test_a_stack_form_that_cannot_hold_the_call_is_refused():
+    with pytest.raises(N.OmniCodecError):
+        plan_stack_shapes(batch=1, length=1000, dilations=(1,), form=N.STACK_FORM_ROWS128 + 1)
+    for kw in (dict(length=300, dilations=(1, 3, 9), form=N.STACK_FORM_SWEEP),      # one tile
+               dict(length=2000, dilations=(1, 1, 3, 9), form=N.STACK_FORM_SWEEP),  # four units
+               dict(length=2000, dilations=(10,), form=N.STACK_FORM_SWEEP),         # halo past the guard
+               dict(length=2000, dilations=(10, 9), form=N.STACK_FORM_ROWS128)):    # 114 halo rows of 128
+        with pytest.raises(N.OmniCodecError) as e:
+            plan_stack_shapes(batch=1, **kw)
+        assert e.value.status == N.UNSUPPORTED
