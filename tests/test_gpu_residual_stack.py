@@ -17,6 +17,7 @@ from sglang_omni_amd.kernels.conv import (
     ResidualUnitWeights,
     fused_conv,
     pack_conv1d,
+    plan_stack_shapes,
     residual_stack,
     stack_coefficients,
 )
@@ -89,8 +90,8 @@ def test_residual_stack_equals_one_launch_per_unit_bitwise(gpu, batch, length, d
 @pytest.mark.parametrize("dilations", [(1, 3, 9), (2,)])
 def test_residual_stack_fp8_weights_equal_one_launch_per_unit_bitwise(gpu, batch, length,
                                                                       dilations):
-    """E4M3 weights: the stack (tiled form for short rows, the sweep for long ones, the weights'
-    bytes staged by LDS DMA and widened when read) against one launch per unit."""
+    """E4M3 weights (their bytes staged by LDS DMA and widened when read) against one launch per
+    unit."""
     units, out_a, out_b = make_units(dilations, gpu, fp8=True, seed=3 + length)
     gen = torch.Generator().manual_seed(1)
     x = (torch.randn(batch, length, C, generator=gen) * 0.3).to(gpu)
@@ -222,15 +223,35 @@ def test_residual_stack_precomputed_coefficients_give_the_same_bits(gpu, fp8, di
                        coef_table=table[:-1])
 
 
-@pytest.mark.parametrize("batch,length", [
-    (1, 301), (1, 345), (1, 4000),       # 128 staged rows: the halo of the first tiles past position 0
-    (1, 12000), (3, 5000), (16, 1500),   # 256 staged rows
-    (100, 2000), (1, 100001),            # the sweep: three tiles a workgroup, an odd length
+FORMS = {"sweep": N.STACK_FORM_SWEEP, "384": N.STACK_FORM_ROWS384, "256": N.STACK_FORM_ROWS256,
+         "128": N.STACK_FORM_ROWS128}
+
+
+def unit_launches(x, units, out_a, out_b, pools, kw):
+    """The units one launch each over the operand's bits, the stream kept in float32."""
+    ref = x.float()
+    u = identity_operand(ref, units[0].in_a, units[0].in_b)
+    for k, unit in enumerate(units):
+        a, b = (units[k + 1].in_a, units[k + 1].in_b) if k + 1 < len(units) else (out_a, out_b)
+        nxt, total = torch.empty_like(u), torch.empty_like(ref)
+        fused_conv(u, unit.conv1, nxt, second=unit.conv2, mid_activation=N.ACT_SNAKE,
+                   mid_a=unit.mid_a, mid_b=unit.mid_b, residual=ref, sum_out=total,
+                   activation=N.ACT_SNAKE, act_a=a, act_b=b, history=pools[k], **kw)
+        u, ref = nxt, total
+    return u, ref
+
+
+@pytest.mark.parametrize("batch,length,form", [
+    (1, 301, "384"),                                  # one whole row
+    (1, 345, "128"), (1, 4000, "128"), (1, 12000, "128"),  # the halo of the first tiles past position 0
+    (3, 5000, "256"), (1, 30001, "256"), (16, 1500, "256"), (1, 100001, "384"),
+    (100, 2000, "sweep"), (100, 2001, "sweep"), (1, 300001, "sweep"),
 ])
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("cold", [True, False])
-def test_every_form_of_long_rows_equals_one_launch_per_unit(gpu, batch, length, fp8, cold):
+def test_every_form_of_long_rows_equals_one_launch_per_unit(gpu, batch, length, form, fp8, cold):
     """The forms the launcher picks by size, with slot histories read (or zeros) and written."""
+    assert plan_stack_shapes(batch=batch, length=length, dilations=(1, 3, 9), fp8=fp8)[0] == FORMS[form]
     units, out_a, out_b = make_units((1, 3, 9), gpu, fp8=fp8, seed=11)
     gen = torch.Generator(device=gpu).manual_seed(length)
     x = (torch.randn(batch, length, C, generator=gen, device=gpu) * 0.3).half()
@@ -242,14 +263,85 @@ def test_every_form_of_long_rows_equals_one_launch_per_unit(gpu, batch, length, 
     got = [p.clone() for p in pools]
     residual_stack(x, units, out, out_a, out_b, histories=got, **kw)
     want = [p.clone() for p in pools]
-    ref = x.float()
-    u = identity_operand(ref, units[0].in_a, units[0].in_b)
-    for k, unit in enumerate(units):
-        a, b = (units[k + 1].in_a, units[k + 1].in_b) if k < 2 else (out_a, out_b)
-        nxt, total = torch.empty_like(u), torch.empty_like(ref)
-        fused_conv(u, unit.conv1, nxt, second=unit.conv2, mid_activation=N.ACT_SNAKE,
-                   mid_a=unit.mid_a, mid_b=unit.mid_b, residual=ref, sum_out=total,
-                   activation=N.ACT_SNAKE, act_a=a, act_b=b, history=want[k], **kw)
-        u, ref = nxt, total
+    u, _ = unit_launches(x, units, out_a, out_b, want, kw)
     assert torch.equal(out, u)
     assert all(torch.equal(p, q) for p, q in zip(got, want))
+
+
+@pytest.mark.parametrize("form", list(FORMS))
+@pytest.mark.parametrize("batch,length", [
+    (1, 3001),   # the sweep: segments of three tiles, the last short
+    (3, 1003),   # two tiles and a few rows
+    (300, 361),  # more rows than CUs, one ragged segment each
+    (37, 12),    # several rows to a tile
+])
+@pytest.mark.parametrize("dilations", [(1, 3, 9), (4,)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_each_form_with_every_output(gpu, form, batch, length, dilations, fp8):
+    """Each form by name: x_out beside out, the coefficient table, the fused final conv with the
+    units' outputs kept or not and with every history, float32 and float16 streams."""
+    if form == "sweep" and length == 12:
+        return  # (whole rows: the sweep refuses them)
+    units, out_a, out_b = make_units(dilations, gpu, fp8=fp8, seed=length)
+    w, b = final_conv_weights(gpu, seed=length)
+    gen = torch.Generator(device=gpu).manual_seed(batch)
+    x32 = torch.randn(batch, length, C, generator=gen, device=gpu) * 0.3
+    pools = [torch.randn(batch, 2, 6 * d, C, generator=gen, device=gpu).bfloat16() for d in dilations]
+    final_pool = torch.randn(batch, 2, 6, C, generator=gen, device=gpu).bfloat16()
+    kw = dict(slot_index=torch.arange(batch, device=gpu).flip(0).contiguous(),
+              slot_parity=torch.arange(batch, device=gpu) % 2, history_cold=False)
+    table = stack_coefficients(units, out_a, out_b)
+    for x in (x32, x32.half()):
+        want_pools = [p.clone() for p in pools]
+        u, ref = unit_launches(x, units, out_a, out_b, want_pools, kw)
+        expected = torch.empty(batch, 1, length, device=gpu)
+        want_final = final_pool.clone()
+        single_output_conv(u, w, b, expected, activation=N.ACT_TANH, left_pad=6, history=want_final, **kw)
+        waves = []
+        for coef, keep, has_final in ((None, True, False), (table, True, True), (None, False, True)):
+            got_pools, got_final = [p.clone() for p in pools], final_pool.clone()
+            out = torch.empty(batch, length, C, dtype=torch.bfloat16, device=gpu) if keep else None
+            x_out = torch.empty_like(x) if keep else None
+            final = None
+            if has_final:
+                waves.append(torch.full((batch, 1, length), float("nan"), device=gpu))
+                final = FinalConv(w, b, N.ACT_TANH, waves[-1], got_final)
+            residual_stack(x, units, out, out_a, out_b, x_out=x_out, histories=got_pools, final=final,
+                           coef_table=coef, form=FORMS[form], **kw)
+            assert all(torch.equal(p, q) for p, q in zip(got_pools, want_pools))
+            if keep:
+                assert torch.equal(out, u) and torch.equal(x_out, ref.to(x.dtype))
+            if has_final:
+                assert torch.equal(got_final, want_final)
+        assert torch.equal(waves[0], waves[1])
+        # the same products as the separate conv's in another float32 order (672 of them)
+        torch.testing.assert_close(waves[0], expected, rtol=0, atol=2e-6)
+
+
+@pytest.mark.parametrize("form", ["sweep", "256", "128"])
+@pytest.mark.parametrize("splits", [(994, 5, 601, 400), (700, 1300)])
+def test_each_form_streams_a_row_in_chunks(gpu, form, splits):
+    """Chunks through the histories (a chunk too short for the form takes the launcher's) equal the
+    whole rows of the launcher's form."""
+    units, out_a, out_b = make_units((1, 3, 9), gpu, seed=17)
+    w, b = final_conv_weights(gpu, seed=4)
+    batch, length = 3, sum(splits)
+    gen = torch.Generator().manual_seed(9)
+    x = (torch.randn(batch, length, C, generator=gen) * 0.3).to(gpu)
+    whole = torch.empty(batch, 1, length, device=gpu)
+    residual_stack(x, units, None, out_a, out_b, final=FinalConv(w, b, N.ACT_TANH, whole))
+    hists = [torch.zeros(5, 2, 6 * d, C, dtype=torch.bfloat16, device=gpu) for d in (1, 3, 9)]
+    fhist = torch.zeros(5, 2, 6, C, dtype=torch.bfloat16, device=gpu)
+    parity = torch.zeros(5, dtype=torch.int64, device=gpu)
+    slot_index = torch.tensor([4, 1, 2], device=gpu)
+    parts, start = [], 0
+    for n, size in enumerate(splits):
+        wave = torch.empty(batch, 1, size, device=gpu)
+        residual_stack(x[:, start:start + size].contiguous(), units, None, out_a, out_b, histories=hists,
+                       slot_index=slot_index, slot_parity=parity, history_cold=n == 0,
+                       final=FinalConv(w, b, N.ACT_TANH, wave, fhist),
+                       form=FORMS[form] if size > 384 else N.STACK_FORM_AUTO)
+        parity[slot_index] += 1
+        parts.append(wave)
+        start += size
+    assert torch.equal(torch.cat(parts, dim=-1), whole)
