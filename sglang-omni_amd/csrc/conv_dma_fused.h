@@ -470,11 +470,12 @@ struct FusedDmaConfig {
            p.weight2 != nullptr && p.mix_a == nullptr && FusedDmaSize<3>::fits(p);
   }
 
-  // The tile of 64 TP positions: the least time at one workgroup per CU, its measured time (20, 28.5
-  // and 36 us; the weight stages, which are the same for each, keep it from shrinking with the
-  // tile) times its rounds. us at TP = 1 / 2 / 3: 15 360 positions 24 / 30 / 37, 30 720 44 / 32 /
-  // 39, 60 036 82 / 58 / 73 (313 tiles of 192 in two rounds, the second a fifth full), 80 000
-  // 103 / 84 / 74, 245 760 315 / 235 / 199 (each with its DMA sent at the stage's start).
+  // The tile of 64 TP positions: the least time at one workgroup per CU, 20, 28.5 and 36 us (the
+  // weight stages, which are the same for each, keep it from shrinking with the tile) times its
+  // rounds. us at TP = 1 / 2 / 3: 16 384 positions 22 / 29 / 35, 32 768 43 / 34 / 39, 60 036 79 / 62
+  // / 71 (313 tiles of 192 in two rounds, the second a fifth full), 80 000 98 / 83 / 72, 245 760 308 /
+  // 246 / 208. A round costs 19 to 22, 24 to 34 and 30 to 41 us as it fills; at 32 sizes from 60 to
+  // 245 760 positions the three numbers, from the middle of those, choose the fastest of the three.
   static constexpr double kUs[3] = {20, 28.5, 36};
   static int tp(const ConvParams& p, double* us) {
     const int64_t wgs[3] = {FusedDmaSize<1>::workgroups(p), FusedDmaSize<2>::workgroups(p),

@@ -8,9 +8,10 @@
 // equals its whole decode. What differs is how the operands arrive:
 //
 //   * a wave owns 16 output columns and 16 TP positions, and reads its columns' weights straight
-//     from memory into the MFMA's operand registers, D - 1 groups of GC chunks ahead (35 to 42
-//     loads of 1 KiB in flight a wave), with no barrier and no LDS on the way: the weights, which
-//     nobody else in the workgroup needs, are what such a call is bound by;
+//     from memory into the MFMA's operand registers, D - 1 groups of GC chunks ahead (GC x taps
+//     loads of 1 KiB a group: 21 in flight a wave at one tap, 36 at two, 35 at seven, 7 in the
+//     residual unit, whose twelve waves share a workgroup), with no barrier and no LDS on the way:
+//     the weights, which nobody else in the workgroup needs, are what such a call is bound by;
 //   * the tile's input rows (positions plus halos) of every channel that fits the LDS are staged
 //     once, by LDS DMA, before the first MFMA (one slab for the decoders' layers at one to a few
 //     row segments; more slabs, each behind a barrier, otherwise).
@@ -24,7 +25,8 @@
 // Measured, us per launch with weights from the Infinity Cache, LDS-DMA tile -> this kernel: at 32
 // positions (4 frames of one stream in block 0) 768 channels k = 7 d = 9 59.7 -> 11.3, k = 1 12.6 ->
 // 5.1; up conv 1536 -> 6144 columns at 4 positions 29.4 -> 11.2; 384 channels at 256 positions k =
-// 7 24.6 -> 8.8, k = 1 10.9 -> 4.6; the 192-channel unit at 1 280 positions 35.7 -> 16.9. The
+// 7 24.6 -> 8.8, k = 1 10.9 -> 4.6; the 192-channel unit at 1 280 positions 35.7 -> 16.6 (the
+// LDS-DMA unit's tiles of 64 positions: 19.1). The
 // crossing lies near 1 000 to 2 000 positions at 768 channels and 4 000 to 8 000 at 192.
 #pragma once
 
@@ -485,7 +487,7 @@ struct SmallUnitConfig {
   static int64_t workgroups(const ConvParams& p) {
     return ((int64_t)p.batch * p.length + Tile::BP - 1) / Tile::BP;
   }
-  // 16.9 us a round (36 us a round of 192 positions per CU in the LDS-DMA form)
+  // 16.4 to 18.9 us a round as it fills (18.6 to 22 in the LDS-DMA form's tiles of 64 positions)
   static double microseconds(const ConvParams& p) { return 17.0 * ((workgroups(p) + 255) / 256); }
   static int launch(ConvParams p, hipStream_t stream) {
     p.p_tiles = (int)workgroups(p);
