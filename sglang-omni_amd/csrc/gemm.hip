@@ -420,13 +420,20 @@ int64_t tiles_of(int64_t rows, int64_t n, int bm, int bn) {
   return ((rows + bm - 1) / bm) * ((n + bn - 1) / bn);
 }
 
+// Compute units of the device, asked once per process (asking takes 0.17 us of a launch's 3.5); 256
+// (MI355X) when the query fails.
 int compute_units() {
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      cus <= 0)
-    return 256;
-  return cus;
+  static const int cached = [] {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        cus <= 0) {
+      (void)hipGetLastError();
+      return 256;
+    }
+    return cus;
+  }();
+  return cached;
 }
 
 bool aligned_to(const void* ptr, int bytes) {
