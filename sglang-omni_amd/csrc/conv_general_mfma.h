@@ -201,15 +201,14 @@ __global__ void __launch_bounds__(kThreads) conv_general_mfma_kernel(const MfmaP
                                     (uint32_t)((j0 + k * j_step) * (int64_t)w_j)
                               : kOutOfRange;
   }
-  // stage (chunk c, tap group tg); the pieces past the rows it reads are left alone
+  // stage (chunk c, tap group tg)
   auto load_stage = [&](int c, int tg) __attribute__((always_inline)) {
     const int c0 = c * KC, tap0 = tg * gt, count = min(gt, nt - tap0);
     if (tap_groups > 1) place_rows(tap0, count);
-    const int x_pieces = stage_rows(count) * 4;
     const uint32_t xbase = (uint32_t)c0 * x_c;
 #pragma unroll
     for (int i = 0; i < Tile::X_PIECES; ++i)
-      if (i * kThreads < x_pieces) xr[i].load(x_rsrc, xoff[i], xbase, x_c, cin_g - c0 - xq);
+      xr[i].load(x_rsrc, xoff[i], xbase, x_c, cin_g - c0 - xq);
     const int pieces = count * BCO * 4;
     const uint32_t wbase = (uint32_t)c0 * w_c + (uint32_t)(tap0 * j_step) * w_j;
 #pragma unroll
