@@ -255,21 +255,25 @@ int omni_conv1d_fused_with(const omni_conv_args* args, int kernel, int config,
  * pre-transformer, `F.linear` in sglang_omni/models/qwen3_omni/components/code2wav.py:266,311,
  * 318,322, and of the ConvNeXt blocks' pointwise convs, incremental_codec.py:174-175), or of a
  * k = 7 conv with few output positions (a decoder's input conv over a streaming step, the
- * `CausalConvNet` of modded_dac.py:566-572): the LDS-DMA kernel runs k_splits slices of the
- * 32-channel chunks of each tile (the k = 7 form staging its history rows per slice and writing
- * the new history of its own chunks), each writing its float32 partial tile [positions][n_cols]
- * into `workspace` (k_splits * batch * length * n_cols floats, 16-byte aligned), then a
- * reduction sums the slices in slice order and applies the bias, the output activation and the
- * bf16 / float32 store. The summation order depends on (c_in, taps, k_splits) only, never on the
- * row count, so a caller that fixes k_splits per layer gets the same bits for a row whatever
- * batch it runs in. Takes: taps = 1 or 7, a bf16 operand without in_activation, bf16 weights,
- * history (k = 7), activation NONE, SNAKE or LEAKY_RELU; no weight2, residual, mix or sum_out;
- * c_in a multiple of 32 * k_splits. k_splits = 1 is omni_conv1d_fused. kernel / config as in
- * omni_conv1d_fused_with (OMNI_CONV_KERNEL_AUTO / 0, or OMNI_CONV_KERNEL_DMA and an entry of its
- * list). k_splits > 1 runs on the LDS-DMA family only: a call that none of its split tiles can
- * hold (e.g. k = 7 over many rows of a few positions each, whose history rows overflow the
- * tile's staged rows) returns OMNI_ERR_UNSUPPORTED before any launch and leaves out untouched;
- * the caller then runs the conv unsplit (omni_conv1d_fused).
+ * `CausalConvNet` of modded_dac.py:566-572): every output is k_splits sums, each over one slice of
+ * the 32-channel chunks (of c_in / k_splits channels) from zero, added up in slice order; then the
+ * bias, the output activation and the bf16 / float32 store. The LDS-DMA kernel runs the slices as
+ * workgroups of their own (the k = 7 form staging its history rows per slice and writing the new
+ * history of its own chunks), each writing its float32 partial tile [positions][n_cols] into
+ * `workspace` (k_splits * batch * length * n_cols floats, 16-byte aligned), and a reduction launch
+ * sums them. The small-call kernel (k = 7) runs a tile's slices one after another in one workgroup
+ * and adds them up in registers: the same bits, no second launch, and `workspace`, which every
+ * call supplies, is left as it was. The summation order depends on (c_in, taps, k_splits) only,
+ * never on the row count, so a caller that fixes k_splits per layer gets the same bits for a row
+ * whatever batch it runs in. Takes: taps = 1 or 7, a bf16 operand without in_activation, bf16
+ * weights, history (k = 7), activation NONE, SNAKE or LEAKY_RELU; no weight2, residual, mix or
+ * sum_out; c_in a multiple of 32 * k_splits. k_splits = 1 is omni_conv1d_fused. kernel / config as
+ * in omni_conv1d_fused_with: OMNI_CONV_KERNEL_AUTO / 0 (the small-call kernel where it is the
+ * faster one, else the LDS-DMA kernel), or OMNI_CONV_KERNEL_DMA and an entry of its list. No other
+ * family runs k_splits > 1: a call that none of the split tiles can hold (e.g. k = 7 over many
+ * rows of a few positions each, whose history rows overflow the tile's staged rows) returns
+ * OMNI_ERR_UNSUPPORTED before any launch and leaves out untouched; the caller then runs the conv
+ * unsplit (omni_conv1d_fused).
  */
 int omni_conv1d_splitk(const omni_conv_args* args, int64_t k_splits, float* workspace,
                        int64_t workspace_bytes, int kernel, int config, omni_stream_t stream);
