@@ -18,12 +18,14 @@ int launch_dma_taps1(const ConvParams& p, bool fp8, Choice& ch, hipStream_t stre
                             DmaConfig<2, 4, 6, 3, 192, 1, 2, false, true>,
                             DmaConfig<2, 4, 3, 3, 192, 1, 3, false, true>,
                             DmaConfig<1, 8, 6, 2, 256, 1, 2, false, true>>(p, ch, stream);
-  // (measured in one round, us at 24 / 12 chunks: 25 / 19.5, 27.5 / 21, 19 / 14.5, 22 / 17)
+  // (measured in one round, us at 24 / 12 chunks: 25 / 19.5, 27.5 / 21, 19 / 14.5, 22 / 17; the third
+  // at 48 chunks 28.4, where 0.45 a chunk had 1536 -> 1536 columns at 2 050 to 3 000 positions take
+  // the 96 x 256 tile of the smaller list, 30.0)
   return launch_least<DmaConfig<4, 4, 3, 3, 192, 1, 2>,
                       DmaConfig<2, 4, 6, 3, 192, 1, 2>,
                       DmaConfig<2, 4, 3, 3, 192, 1, 3>,
                       DmaConfig<1, 8, 6, 2, 256, 1, 2>>(
-      p, {{13.5, 0.5}, {15, 0.54}, {9, 0.45}, {12, 0.47}}, ch, stream);
+      p, {{13.5, 0.5}, {15, 0.54}, {9.2, 0.4}, {12, 0.47}}, ch, stream);
 }
 
 }  // namespace omni_conv

@@ -150,6 +150,14 @@ def test_what_no_tile_serves_the_small_kernel_does_not_either():
     assert loaded.kernel == N.CONV_KERNEL_FUSED_UNIT
 
 
+@pytest.mark.parametrize("positions", [2049, 2500, 2905, 3000])
+def test_deep_one_tap_layers_take_the_tile_of_192_positions(positions):
+    """1536 -> 1536 columns, us: 96 x 192 28.4, the smaller list's 96 x 256 30.0 (up to 2 048
+    positions one round of its 96 x 128 tiles, 22.7)."""
+    plan = plan_shapes(batch=1, length=positions, c_in=1536, n_cols=1536, c_out=1536, taps=1)
+    assert plan.kernel == N.CONV_KERNEL_DMA and plan.config == 3
+
+
 @pytest.mark.parametrize("batch,length,form", [
     # the form measured fastest of the four (us: sweep / 384 / 256 / 128 rows)
     (1, 310, N.STACK_FORM_ROWS128),       # 84 / 52 / 41 / 29
