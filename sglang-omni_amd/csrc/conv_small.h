@@ -443,11 +443,16 @@ struct SmallConfig {
   // frames; within 25 %): what a workgroup reads at 80 KB per us, its steps' instructions, its
   // epilogue, times the workgroups of the fullest CU (also where its LDS holds several at once: 288
   // of 4 waves at 768 -> 3072 columns, two taps, 96 positions take 19.6 us, 192 of 2 waves 12.1).
+  // A CU holds eight waves of one tap (two a SIMD): further workgroups start, and wait for their
+  // first loads, when those are done (192 -> 192 columns, 4 waves of 32 positions: 237 workgroups
+  // 6.1 us, 471 7.1, 564 10.2; the LDS-DMA tile of 96 x 192 9.5).
   static double microseconds(const ConvParams& p) {
     const double rows = (double)rows_needed(p), steps = (double)(p.c_in / kChunk) * TAPS;
     const double us = (steps * Tile::BCO * Tile::ES + rows * p.c_in * 2) / 80e3 +
                       TP * (0.018 * steps + 0.4);
-    return 3 + us * (double)((workgroups(p) + 255) / 256);
+    const int64_t per_cu = (workgroups(p) + 255) / 256;
+    const int64_t starts = TAPS == 1 ? (per_cu * NW + 7) / 8 : 1;
+    return 3.0 * starts + us * per_cu;
   }
   static int launch(ConvParams p, hipStream_t stream) {
     const int64_t positions = (int64_t)p.batch * p.length;

@@ -150,6 +150,17 @@ def test_what_no_tile_serves_the_small_kernel_does_not_either():
     assert loaded.kernel == N.CONV_KERNEL_FUSED_UNIT
 
 
+@pytest.mark.parametrize("c_in,n_cols", [(96, 192), (192, 192), (192, 768), (384, 384)])
+def test_one_tap_small_calls_start_every_workgroup_at_once(c_in, n_cols):
+    """A CU holds eight waves of the one-tap small kernel; a call whose workgroups are more starts
+    some of them after the others' end and is slower than the LDS-DMA tiles."""
+    for positions in range(100, 12000, 100):
+        plan = plan_shapes(batch=1, length=positions, c_in=c_in, n_cols=n_cols, c_out=n_cols, taps=1)
+        if plan.kernel == N.CONV_KERNEL_SMALL:
+            waves = (1, 2, 4)[(plan.config - 1) % 3]
+            assert -(-plan.workgroups // 256) * waves <= 8, (positions, plan)
+
+
 @pytest.mark.parametrize("positions", [2049, 2500, 2905, 3000])
 def test_deep_one_tap_layers_take_the_tile_of_192_positions(positions):
     """1536 -> 1536 columns, us: 96 x 192 28.4, the smaller list's 96 x 256 30.0 (up to 2 048
