@@ -519,9 +519,12 @@ int launch_small_list(const ConvParams& p, double than, Choice& ch, hipStream_t 
   int pick = -1;
   if (ch.force == 0) {
     than /= 1.15;
-    const double us[n] = {(Cfgs::fits(p) ? Cfgs::microseconds(p) : 1e30)...};
-    for (int i = 0; i < n; ++i)
-      if (us[i] < than) pick = i, than = us[i];
+    double (*const microseconds[n])(const ConvParams&) = {&Cfgs::microseconds...};
+    for (int i = 0; i < n; ++i) {
+      if (!fits[i]) continue;
+      const double us = microseconds[i](p);
+      if (us < than) pick = i, than = us;
+    }
     if (pick < 0) return OMNI_ERR_UNSUPPORTED;
   }
   return choose_and_launch(ch, n, fits, wgs, launch, pick, p, stream);
