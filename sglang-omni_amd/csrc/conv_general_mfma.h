@@ -293,8 +293,8 @@ __global__ void __launch_bounds__(kThreads) conv_general_mfma_kernel(const MfmaP
   }
 
   // A tap outside the row adds nothing, but the matrix cores multiply its staged zeros all the same,
-  // which an infinite or NaN weight turns into NaN: in the tiles at a row's ends an output that is
-  // not finite is summed again, without the taps outside (`again`: bit 4 TCO u + 4 c + e).
+  // which an infinite or NaN weight turns into NaN: at a row's ends an output with a tap outside that
+  // is not finite is summed again, without the taps outside (`again`: bit 4 TCO u + 4 c + e).
   const int d_last = d0 + (nt - 1) * d_step;
   const bool edge = u0 * p.u_step + min(d0, d_last) < 0 ||
                     (min(u0 + BP, p.u_count) - 1) * p.u_step + max(d0, d_last) >= (int)g.length_in;
@@ -302,12 +302,15 @@ __global__ void __launch_bounds__(kThreads) conv_general_mfma_kernel(const MfmaP
   static_assert(4 * TCO * TP <= 64, "a bit for each of a lane's outputs");
   if (edge) {
 #pragma unroll
-    for (int u = 0; u < TP; ++u)
+    for (int u = 0; u < TP; ++u) {
+      const int pos = (u0 + u_wave + u * 16 + lrow) * p.u_step;
+      const bool outside = pos + min(d0, d_last) < 0 || pos + max(d0, d_last) >= (int)g.length_in;
 #pragma unroll
       for (int c = 0; c < TCO; ++c)
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          if (!__builtin_isfinite(acc[c][u][e])) again |= 1ull << (4 * (TCO * u + c) + e);
+          if (outside && !__builtin_isfinite(acc[c][u][e])) again |= 1ull << (4 * (TCO * u + c) + e);
+    }
   }
 
   // lane: position lrow of a group of 16, output channels 4 lq .. 4 lq + 3 of 16
